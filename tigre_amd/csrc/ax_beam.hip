@@ -1,12 +1,12 @@
-// Beam-staged Siddon forward projector for gfx950.
+// Beam-staged forward projectors for gfx950.
 //
-// A 1024-thread workgroup traces the rays of a 16 x 16 detector tile in up to
-// four views that share a principal axis P (the horizontal axis, x or y, along
+// A 1024-thread workgroup traces the rays of a detector tile (1024 rays: 32 x 8 pixels in four views, 64 x 16
+// in one, ...) in up to four views that share a principal axis P (the horizontal axis, x or y, along
 // which their rays advance fastest) and its direction.  Their rays form a thin
 // beam.  The workgroup sweeps the volume along P in slabs of a few planes; for
 // each slab it copies the box of voxels the beam crosses into LDS (16-byte
 // loads of rows of a re-laid-out copy of the volume), and every ray walks its
-// Siddon crossings inside the slab reading voxels from LDS.  The gathers of
+// voxels inside the slab from LDS.  The gathers of
 // the walk thus never reach the texture/L1 path, which bounds a gather-driven
 // walk; the slab copies are coalesced and are shared by the 1024 rays.
 //
@@ -20,7 +20,8 @@
 // copies.
 //
 // Planning: every wavefront evaluates the 16 corner rays of the tile (four
-// corners in each view) and computes the box origins of a share of the slabs;
+// corners in each view) and computes the box origins of a share of the slabs (Siddon skips the slabs
+// before and after the volume);
 // the box extents, maxed over the slabs, are the same for the whole sweep, so
 // a ray's LDS offset carries from one slab to the next by a uniform shift.
 // Slabs are double-buffered: slab s + 1 streams into LDS by direct
@@ -36,9 +37,7 @@ namespace tigre {
 
 namespace {
 
-constexpr int kBeamTile = 16;       // detector pixels per tile edge
-constexpr int kBeamViews = 4;       // views per workgroup
-constexpr int kBeamThreads = kBeamViews * kBeamTile * kBeamTile;
+constexpr int kBeamThreads = 1024;
 constexpr int kSlabCap = 9216;      // floats per LDS slab buffer (two per workgroup)
 constexpr int kSlabPlanesMax = 8;   // principal planes per slab, at most (the tunable limit is <= this)
 
@@ -70,8 +69,11 @@ __device__ __forceinline__ float corner_max(float x) {
 // upper interpolation tap.  Clipped to -1 .. n + tap (no walk or tap leaves
 // it: a sample clamped to the face n reads the zero tap n + 1 with weight 0);
 // a0 is aligned down to 4 for 16-byte rows.
+// `rim`: a line may leave the volume in the planes; `out`: all of them stay outside it (a 64th of a voxel
+// covers the rounding of the lines).
 struct BoxExtent {
     int a0, a1, z0, z1;
+    bool rim, out;
 };
 __device__ inline BoxExtent beam_extent(int lo, int hi, float cA, float kA, float cz, float kz, int nA, int nz,
                                         int tap) {
@@ -80,11 +82,14 @@ __device__ inline BoxExtent beam_extent(int lo, int hi, float cA, float kA, floa
     const float Z0 = fmaf(kz, p0, cz), Z1 = fmaf(kz, p1, cz);
     float amin = corner_min(fminf(A0, A1)), amax = corner_max(fmaxf(A0, A1));
     float zmin = corner_min(fminf(Z0, Z1)), zmax = corner_max(fmaxf(Z0, Z1));
+    constexpr float kTol = 1.0f / 64.0f;
+    BoxExtent e;
+    e.rim = amin < kTol || amax > (float)nA - kTol || zmin < kTol || zmax > (float)nz - kTol;
+    e.out = amax < -kTol || amin > (float)nA + kTol || zmax < -kTol || zmin > (float)nz + kTol;
     amin = fminf(fmaxf(amin, -2.0f), (float)nA + 1.0f);
     amax = fminf(fmaxf(amax, -2.0f), (float)nA + 1.0f);
     zmin = fminf(fmaxf(zmin, -2.0f), (float)nz + 1.0f);
     zmax = fminf(fmaxf(zmax, -2.0f), (float)nz + 1.0f);
-    BoxExtent e;
     e.a0 = max((int)floorf(amin) - 1, -1) & ~3;
     e.a1 = min((int)floorf(amax) + 1 + tap, nA + tap);
     e.z0 = max((int)floorf(zmin) - 1, -1);
@@ -198,6 +203,124 @@ __device__ inline bool walk(RayWalk& r, const float* __restrict__ base, unsigned
     return tm >= T;
 }
 
+// Plane walk of the Siddon projector: one principal cell (one plane of voxels) per step.
+//
+// Along the sweep a ray advances one voxel in P per step and at most one voxel in A and in z (slopes
+// below 1), so a cell holds at most two crossings and three segments.  A and z are taken in mirrored
+// indices that increase along the sweep and in fixed point with 32 fraction bits, A(s) = A0 + s kA, s counted in
+// cells from cell -1.  In the cell the ray enters at fraction f of an A voxel it crosses the next A plane
+// at the fraction tA = min((1 - f) / kA, 1) of the cell, and likewise in z.  With t1 <= t2 the two
+// sorted, the cell adds
+//     t1 v0 + (t2 - t1) v1 + (1 - t2) v2,
+// v0 the entry voxel, v1 the one past the first crossing, v2 the exit voxel.  Whether an axis crosses is the
+// carry of the fraction's addition, so voxel and position cannot part, a voxel that is not crossed is
+// not read, and the sums do not depend on how a sweep is cut into slabs.  The slope in 32 bits puts a ray
+// at most 2^-33 voxel a cell off its line (1e-7 after 1024 cells); an FP32 crossing time is
+// off by 3e-5 voxel there.
+//
+// The step has no branch and no division, about 20 VALU instructions and (planes at a constant LDS stride, so
+// the plane is an immediate of the read) three LDS reads, all lanes in step; the crossing walk above takes
+// one crossing per step, about 17 instructions each, 1.6 times a cell on average, and its lanes leave a slab
+// at different steps.  It stays for rays with a slope of 1 or more (detector tiles that look across the 45
+// degree diagonal, about 4 % of them at a fan angle of 15 degrees).
+//
+// Measured at 512^3 voxels, 512^2 pixels, 360 views: 25.3 ms, 36.5 ms with the crossing walk alone; 23 VALU
+// instructions per ray and plane (33.8 before), 3.4 cycles each (most pairs of an FMA and another operation
+// issue together), and 5 TB/s of copies.  What is scalar or serial in the slab loop counts as much:
+// with the slabs' addresses formed in the loop instead of read from a table the same walk took 30.5 ms.  Two rays per lane
+// with half the wavefronts moved 40 % less and were slower (33 ms).
+struct PlaneRay {
+    unsigned long long A0, z0;  // mirrored A and z at the start of cell -1, 2^-32 voxel
+    unsigned kA, kz;            // slopes, 2^-32 voxel
+    float iA, iz;               // their reciprocals
+    int dA, dZ;                 // offset step of one (mirrored) index on A (1 or -1) and on z (row steps)
+    unsigned off;               // voxel offset in the current source, as in RayWalk
+    float sum;
+};
+
+// Mirrored position and slope on one axis of the line s0 + r a, from the start of cell -1, which the
+// sweep enters at parameter a0 and leaves da later; a ray parallel to the axis stays inside its voxel
+// (or on the border).
+__device__ __forceinline__ void plane_axis(double s0, double r, double a0, double da, int n, unsigned long long& x0,
+                                           unsigned& k, float& ik, int& step) {
+    double x = s0 + r * a0, slope = r * da;
+    step = 1;
+    if (r == 0.0) x = (s0 > 0.0 && s0 < (double)n) ? floor(s0) + 0.5 : -1.0;
+    if (slope < 0.0) {
+        x = (double)n - x;
+        slope = -slope;
+        step = -1;
+    }
+    const double f = floor(x);
+    x0 = ((unsigned long long)(long long)f << 32) + (unsigned long long)((x - f) * 4294967296.0);
+    k = (unsigned)rint(slope * 4294967296.0);
+    ik = k != 0u ? (float)(1.0 / slope) : 1e30f;
+}
+
+// Offset of the voxel of a ray at the start of cell `first`, in a box of origin (a0, z0) and row length na;
+// positions outside the volume are taken on the border (-1 or n).
+__device__ __forceinline__ unsigned plane_offset(const PlaneRay& r, int first, int a0, int z0, int na, int nA, int nz) {
+    const int iA = min(max((int)((r.A0 + (unsigned long long)r.kA * (unsigned)first) >> 32), -1), nA);
+    const int iz = min(max((int)((r.z0 + (unsigned long long)r.kz * (unsigned)first) >> 32), -1), nz);
+    const int a = r.dA > 0 ? iA : nA - 1 - iA, z = r.dZ > 0 ? iz : nz - 1 - iz;
+    return (unsigned)((z - z0) * na + (a - a0));
+}
+
+// Whether a ray is in the volume in cells first .. first + count - 1: 0 outside in all of them, 2 never
+// further out than the border, 1 else.
+__device__ __forceinline__ int plane_range(const PlaneRay& r, int first, int count, int nA, int nz) {
+    const unsigned long long xA = r.A0 + (unsigned long long)r.kA * (unsigned)first;
+    const unsigned long long xz = r.z0 + (unsigned long long)r.kz * (unsigned)first;
+    const int sA = (int)(xA >> 32), eA = (int)((xA + (unsigned long long)r.kA * (unsigned)count) >> 32);
+    const int sz = (int)(xz >> 32), ez = (int)((xz + (unsigned long long)r.kz * (unsigned)count) >> 32);
+    if (eA < 0 || sA >= nA || ez < 0 || sz >= nz) return 0;
+    return sA >= -1 && eA <= nA && sz >= -1 && ez <= nz ? 2 : 1;
+}
+
+// Cells first .. first + count - 1 of the sweep (at most eight); the ray's voxel is at r.off + slot of
+// `base`, planes PS apart (kPS > 0: this constant).  kRim: a ray of the tile may lie outside the volume
+// here; outside, it stays on the border, whose voxels are 0, and enters with the index that the border is next to.
+template <bool kLds, int kPS, bool kRim>
+__device__ __forceinline__ void plane_cells(PlaneRay& r, const float* __restrict__ base, unsigned slot, unsigned PS,
+                                            int nA, int nz, int first, int count) {
+    constexpr int kSh = kLds ? 2 : 0;  // byte offsets in LDS, element offsets in the staging copy
+    const unsigned long long xA = r.A0 + (unsigned long long)r.kA * (unsigned)first;
+    const unsigned long long xz = r.z0 + (unsigned long long)r.kz * (unsigned)first;
+    unsigned A = (unsigned)xA, z = (unsigned)xz;
+    int iA = (int)(xA >> 32), iz = (int)(xz >> 32);
+    const unsigned dA = (unsigned)r.dA << kSh, dZ = (unsigned)r.dZ << kSh;
+    unsigned off = (r.off + slot) << kSh;
+    const float sA = r.iA * 0x1p-32f, sz = r.iz * 0x1p-32f;
+    float sum = r.sum;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (j >= count) break;  // uniform
+        auto read = [&](unsigned o) {
+            return kLds ? *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (o + (kPS > 0 ? 4 * kPS * j : 0)))
+                        : base[o];
+        };
+        const float tA = __builtin_amdgcn_fmed3f(fmaf((float)A, -sA, r.iA), 0.0f, 1.0f);
+        const float tz = __builtin_amdgcn_fmed3f(fmaf((float)z, -sz, r.iz), 0.0f, 1.0f);
+        bool cA = __builtin_add_overflow(A, r.kA, &A), cz = __builtin_add_overflow(z, r.kz, &z);
+        if (kRim) {
+            const bool inA = (unsigned)(iA + 1) <= (unsigned)nA, inz = (unsigned)(iz + 1) <= (unsigned)nz;
+            iA += cA ? 1 : 0;
+            iz += cz ? 1 : 0;
+            cA = cA && inA;
+            cz = cz && inz;
+        }
+        const unsigned stepA = cA ? dA : 0u, stepz = cz ? dZ : 0u;
+        const unsigned mid = off + (tA < tz ? stepA : stepz), end = off + stepA + stepz;
+        const float t1 = fminf(tA, tz), t2 = fmaxf(tA, tz);
+        sum = fmaf(t1, read(off), sum);
+        sum = fmaf(t2 - t1, read(mid), sum);
+        sum = fmaf(1.0f - t2, read(end), sum);
+        off = kPS > 0 ? end : end + (PS << kSh);
+    }
+    r.off = (off >> kSh) - slot;
+    r.sum = sum;
+}
+
 // Workgroup table entry: views [first, first + count) of the ordered view
 // records share principal axis `principal` and direction `dir`.
 struct BeamGroup {
@@ -206,10 +329,28 @@ struct BeamGroup {
 
 constexpr int kMaxSlabs = 272;
 
+// What the sweep needs of a slab, uniform: the byte offset of its box's lowest corner in the staging copy, the
+// box's origin and whether a ray may lie outside the volume there (rim).
+struct SlabBox {
+    long long src;
+    int a0, z0;  // Siddon: a0 holds the origin's offset a0 + z0 na, z0 the rim flag
+};
+__device__ __forceinline__ SlabBox slab_box(const int4* box, int s) {
+    const int4 v = box[s];
+    SlabBox b;
+    b.src = (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(v.y) << 32) |
+                        (unsigned)__builtin_amdgcn_readfirstlane(v.x));
+    b.a0 = __builtin_amdgcn_readfirstlane(v.z);
+    b.z0 = __builtin_amdgcn_readfirstlane(v.w);
+    return b;
+}
+constexpr int kPlaneStride = kSlabCap / kSlabPlanesMax;  // LDS plane stride of an eight-plane Siddon slab
+
 struct SweepShared {
     float buf[2 * kSlabCap];
-    int2 origin[kMaxSlabs];  // (a0, z0) of each slab box
+    int4 box[kMaxSlabs];     // per slab, see SlabBox (during planning: a0, z0, rim)
     int ext[2];              // box extents na (multiple of 4) and nzb, maxed over the slabs
+    int live[2];             // first and last slab whose box meets the volume (Siddon)
 };
 
 // Per-ray state of the interpolated projector (ray_interpolated_projection.cu
@@ -334,15 +475,17 @@ __device__ inline bool sample_slab(RaySamples& r, const float* __restrict__ base
     return done;
 }
 
-// One workgroup: the rays of a 16 x 16 detector tile in up to four views.
+// One workgroup: the rays of a detector tile in the views of a group.  The tile is cut into units of 16 x 4
+// pixels of one view, one wavefront each, one lane per pixel (see BeamShape).
 // kMode 0: Siddon; 1: trilinear interpolation; 2: nearest-voxel sampling.
 template <int kP, int kMode>
 __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGeom& sg, int nx, int ny, int nz,
                                   const FwdView* __restrict__ views, const BeamGroup& grp, int tile_u, int tile_v,
-                                  int stack, int nU, int nV, long long su, long long sv, long long sview,
+                                  BeamShape shape, int nU, int nV, long long su, long long sv, long long sview,
                                   float* __restrict__ out, double acc, double dvx, double dvy, double dvz,
                                   int max_planes, SweepShared& sh) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nP = kP == 0 ? nx : ny, nA = kP == 0 ? ny : nx;
     const int dir = grp.dir;
     // Siddon visits principal voxels -1 .. nP; samples have lower taps in cells
@@ -350,116 +493,22 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
     const int last_cell = kMode == 0 ? nP : nP - 1;
     const int tap = kMode == 0 ? 0 : 1;
 
-    // ---- the lane's ray (FP64 set-up) ----
-    // Slot s (four wavefronts) traces view first + s of the group in tile
-    // (tile_u, tile_v).  Stacked, the slots trace `stack` tiles of each of the
-    // 4 / stack views a group may hold: two (groups of at most two views), the
-    // tiles (2 tile_u + (s >> 1), tile_v) of view s & 1; four (groups of one
-    // view), the 2 x 2 tiles (2 tile_u + (s & 1), 2 tile_v + (s >> 1)).
-    const int slot = wave >> 2;
-    const int per = 4 / stack;  // views per workgroup
-    auto slot_view = [&](int s) { return grp.first + min(s % per, grp.count - 1); };
-    auto slot_tu = [&](int s) { return stack == 1 ? tile_u : 2 * tile_u + (stack == 2 ? s >> 1 : s & 1); };
-    auto slot_tv = [&](int s) { return stack == 4 ? 2 * tile_v + (s >> 1) : tile_v; };
-    const int u = slot_tu(slot) * kBeamTile + (lane & 15);
-    const int v = slot_tv(slot) * kBeamTile + (wave & 3) * 4 + (lane >> 4);
-    const bool active = slot % per < grp.count && u < nU && v < nV;
-    const FwdView& w = views[slot_view(slot)];
-    RayWalk r;
-    r.sum = 0.0f;
-    RaySamples rs;
-    rs.sum = 0.0f;
-    int state = 0;  // 0: no ray or finished, 1: waiting for the slab of its entry, 2: walking
-    int ip0 = 0, ia0 = 0, iz0 = 0, sx = 0, sy = 0, sz = 0;
-    double len = 0.0;
-    if (active) {
-        const double pv = (double)(nV - 1 - v);  // detector row flip, Siddon_projection.cu:141
-        double sp[3];
-        ray_source(w, u, pv, sp);
-        double rx = ray_dir(w, u, pv, 0);
-        double ry = ray_dir(w, u, pv, 1);
-        double rz = ray_dir(w, u, pv, 2);
-        if (kMode == 0) {
-            if (w.pad[1] != 0.0) parallel_siddon_height(sp, rx, ry, rz, nx, ny);
-            // components below 1e-3 voxel are treated as exactly zero (:155-159)
-            if (fabs(rx) < 1e-3) rx = 0.0;
-            if (fabs(ry) < 1e-3) ry = 0.0;
-            if (fabs(rz) < 1e-3) rz = 0.0;
-            len = sqrt(rx * rx * dvx * dvx + ry * ry * dvy * dvy + rz * rz * dvz * dvz);  // mm (:241, :267)
-            double am = -INFINITY, aM = INFINITY;
-            bool hit = slab(sp[0], rx, nx, am, aM);
-            hit = hit && slab(sp[1], ry, ny, am, aM);
-            hit = hit && slab(sp[2], rz, nz, am, aM);
-            if (hit && am < aM) {  // a ray that misses the volume projects to 0 (:179-180)
-                const Axis ax = axis_setup(sp[0], rx, am);
-                const Axis ay = axis_setup(sp[1], ry, am);
-                const Axis az = axis_setup(sp[2], rz, am);
-                r.tx = r.t0x = ax.t0;
-                r.ty = r.t0y = ay.t0;
-                r.tz = r.t0z = az.t0;
-                r.dtx = ax.dt;
-                r.dty = ay.dt;
-                r.dtz = az.dt;
-                r.kx = r.ky = r.kz = 0.0f;
-                r.T = (float)(aM - am);
-                r.tc = 0.0f;
-                ip0 = kP == 0 ? ax.idx : ay.idx;
-                ia0 = kP == 0 ? ay.idx : ax.idx;
-                iz0 = az.idx;
-                sx = ax.step;
-                sy = ay.step;
-                sz = az.step;
-                state = 1;
-            }
-        } else {
-            // samples per ray and step (ray_interpolated_projection.cu:164-169)
-            const double n = sample_count(w, sqrt(rx * rx + ry * ry + rz * rz), acc);
-            if (n >= 1.0 && n < 1e9) {  // else: degenerate ray (pixel at the source), 0
-                const double st[3] = {rx / n, ry / n, rz / n};
-                // sample range [first, last] of the reference (:182-193), clipped to
-                // the samples strictly inside (-1, n) on every axis (the others are
-                // exactly zero)
-                const double last = (w.cap < n) ? ceil(w.cap) : n;
-                double lo = -INFINITY, hi = INFINITY;
-                const int nn[3] = {nx, ny, nz};
-                bool empty = false;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    if (st[a] == 0.0) {
-                        if (!(sp[a] > -1.0 && sp[a] < (double)nn[a])) empty = true;
-                    } else {
-                        const double a0 = (-1.0 - sp[a]) / st[a], a1 = ((double)nn[a] - sp[a]) / st[a];
-                        lo = fmax(lo, fmin(a0, a1));
-                        hi = fmin(hi, fmax(a0, a1));
-                    }
-                }
-                const double i0 = fmax(w.first, floor(lo));
-                const double i1 = fmin(last, ceil(hi));
-                len = sqrt(st[0] * dvx * st[0] * dvx + st[1] * dvy * st[1] * dvy + st[2] * dvz * st[2] * dvz);
-                if (!empty && i0 <= i1) {
-                    // positions relative to the first sample keep the FP32 loop accurate
-                    rs.qP = (float)(sp[kP] + i0 * st[kP]);
-                    rs.qA = (float)(sp[1 - kP] + i0 * st[1 - kP]);
-                    rs.qz = (float)(sp[2] + i0 * st[2]);
-                    rs.fP = (float)st[kP];
-                    rs.fA = (float)st[1 - kP];
-                    rs.fz = (float)st[2];
-                    rs.m = 0;
-                    rs.count = (int)(i1 - i0) + 1;
-                    state = 2;
-                }
-            }
-        }
-    }
+    // ---- this lane's pixel ----
+    const int upv = shape.units_u * shape.units_v;  // units per view
+    const int edge_u = 16 * shape.units_u, edge_v = 4 * shape.units_v;
+    const int vi = wave / upv, k = wave % upv;
+    const int u = tile_u * edge_u + 16 * (k % shape.units_u) + (lane & 15);
+    const int v = tile_v * edge_v + 4 * (k / shape.units_u) + (lane >> 4);
+    const bool active = vi < grp.count && u < nU && v < nV;
+    const FwdView& w = views[grp.first + min(vi, grp.count - 1)];
 
-    // ---- corner rays of the tile (lanes 0..15 of every wavefront) ----
+    // ---- corner rays of the tile (lanes 0..15 of every wavefront, four per view) ----
     float cA, kA, cz, kz;
     {
         const int c = lane & 15;
-        const int cs = c >> 2;
-        const FwdView& cw = views[slot_view(cs)];
-        const int cu = min(slot_tu(cs) * kBeamTile + ((c & 1) ? kBeamTile - 1 : 0), nU - 1);
-        const int cvv = min(slot_tv(cs) * kBeamTile + ((c & 2) ? kBeamTile - 1 : 0), nV - 1);
+        const FwdView& cw = views[grp.first + min(c >> 2, grp.count - 1)];
+        const int cu = min(tile_u * edge_u + ((c & 1) ? edge_u - 1 : 0), nU - 1);
+        const int cvv = min(tile_v * edge_v + ((c & 2) ? edge_v - 1 : 0), nV - 1);
         const double pv = (double)(nV - 1 - cvv);
         double csrc[3];
         ray_source(cw, cu, pv, csrc);
@@ -476,39 +525,226 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
     // ---- plan: box origins of every slab (in parallel over the wavefronts)
     // and the extents shared by all of them; fewer planes per slab until the
     // box fits an LDS buffer ----
-    int planes = 0, nslabs = 0, na = 0, nzb = 0;
+    int planes = 0, first_slab = 0, nslabs = 0, na = 0, nzb = 0;
     bool staged = false;
     for (int attempt = 0; attempt < 5 && !staged; ++attempt) {
-        const int pl_try = attempt == 0 ? max_planes
-                                        : min(max_planes, attempt == 1 ? 6 : (attempt == 2 ? 4 : (attempt == 3 ? 2 : 1)));
+        int pl_try = attempt == 0 ? max_planes
+                                  : min(max_planes, attempt == 1 ? 6 : (attempt == 2 ? 4 : (attempt == 3 ? 2 : 1)));
+        // Siddon: a constant plane stride, or a power of two of planes
+        if (kMode == 0) pl_try = pl_try >= 8 ? 8 : (pl_try >= 4 ? 4 : (pl_try >= 2 ? 2 : 1));
         const int ns = (last_cell + 2 + pl_try - 1) / pl_try;
         if (ns > kMaxSlabs) continue;
-        if (tid == 0) sh.ext[0] = sh.ext[1] = 0;
+        if (tid == 0) {
+            sh.ext[0] = sh.ext[1] = 0;
+            sh.live[0] = ns;
+            sh.live[1] = -1;
+        }
         __syncthreads();
         for (int s = wave; s < ns; s += kBeamThreads / 64) {
             int lo, hi;
             slab_range(s, pl_try, dir, last_cell, lo, hi);
             const BoxExtent e = beam_extent(lo, hi, cA, kA, cz, kz, nA, nz, tap);
             if (lane == 0) {
-                sh.origin[s] = make_int2(e.a0, e.z0);
+                sh.box[s] = make_int4(e.a0, e.z0, e.rim ? 1 : 0, 0);
+                // (a slab outside the volume can lie between two that meet it: the beams of several views part)
                 atomicMax(&sh.ext[0], (e.a1 - e.a0 + 4) & ~3);
                 atomicMax(&sh.ext[1], e.z1 - e.z0 + 1);
+                if (kMode != 0 || !e.out) {
+                    atomicMin(&sh.live[0], s);
+                    atomicMax(&sh.live[1], s);
+                }
             }
         }
         __syncthreads();
-        na = sh.ext[0];
-        nzb = sh.ext[1];
+        na = __builtin_amdgcn_readfirstlane(sh.ext[0]);
+        nzb = __builtin_amdgcn_readfirstlane(sh.ext[1]);
         if (na * nzb * (pl_try + tap) <= kSlabCap) {
             staged = true;
             planes = pl_try;
-            nslabs = ns;
+            first_slab = __builtin_amdgcn_readfirstlane(sh.live[0]);
+            nslabs = __builtin_amdgcn_readfirstlane(sh.live[1]) + 1;
         }
         __syncthreads();  // ext is reset by the next attempt
     }
 
-    if (!staged) {
-        // The beam's box does not fit an LDS buffer: read the staging copy.
-        if (kMode == 0) {
+    // ---- copies: Siddon planes lie in sweep order at a fixed stride, samples' planes in increasing
+    // order and close ----
+    const int SP = kMode == 0 ? kSlabCap / max(planes, 1) : nzb * na;
+    const bool down = kMode == 0 && dir < 0;  // the first LDS plane is the highest
+    // this thread's quads of a box: row (plane, z) and 4-float column, as a byte offset from the box's lowest
+    // corner (32 bits: a box spans few planes); quads in the pad between planes and after the last copy the corner
+    const int nq4 = max(na >> 2, 1), prow = max(kMode == 0 ? SP >> 2 : nzb * nq4, 1);  // row and plane in quads
+    const int nq = (planes + tap) * prow;                                             // of a full slab
+    constexpr int kLoads = (kSlabCap / 4 + kBeamThreads - 1) / kBeamThreads;
+    unsigned qoff[kLoads];
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+        const int q = tid + j * kBeamThreads;
+        const int pl = q / prow, rest = q - pl * prow;
+        const int zr = rest / nq4, aq = rest - zr * nq4;
+        const bool in = pl < planes + tap && zr < nzb;
+        qoff[j] = in ? 4u * (unsigned)(((down ? planes - 1 - pl : pl) * sg.NZ + zr) * sg.NA + 4 * aq) : 0u;
+    }
+    // the slabs' table, one slab per lane (a short last slab's lowest corner is where a full one's would be)
+    const int cells_total = last_cell + 2;
+    if (staged && tid < nslabs) {
+        int lo, hi;
+        slab_range(tid, planes, dir, last_cell, lo, hi);
+        const int4 e = sh.box[tid];
+        const long long src = ((long long)((down ? hi - planes + 1 : lo) + 1) * sg.NZ + (e.y + 1)) * sg.NA + (e.x + 4);
+        sh.box[tid] = make_int4((int)(4 * src), (int)((4 * src) >> 32), kMode == 0 ? e.y * na + e.x : e.x,
+                                kMode == 0 ? e.z : e.y);
+    }
+    __syncthreads();
+    const int wave_first = wave * 64;
+    const char* stage_bytes = reinterpret_cast<const char*>(stage);
+    // Direct global-to-LDS copies (16 bytes per lane) of slab s: quad q lands
+    // at buf[4 q]; the LDS base of each instruction is uniform per wavefront.
+    auto fetch = [&](int s, long long from) {
+        float* dst = sh.buf + (s & 1) * kSlabCap + 4 * wave_first;
+        const char* src = stage_bytes + from;
+        const int count = cells_total - s * planes;
+        if (count >= planes) {
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (wave_first + j * kBeamThreads < nq)  // uniform
+                    __builtin_amdgcn_global_load_lds(src + qoff[j], dst + 4 * j * kBeamThreads, 16, 0, 0);
+        } else {
+            // a short last slab: its own planes alone
+            const int nqs = (count + tap) * prow;
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (wave_first + j * kBeamThreads < nqs && tid + j * kBeamThreads < nqs && (qoff[j] != 0u || tid + j == 0))
+                    __builtin_amdgcn_global_load_lds(src + qoff[j], dst + 4 * j * kBeamThreads, 16, 0, 0);
+        }
+    };
+    // The slabs one after the other: `cells(s, box, slot)` walks the box of slab s, staged at buf[slot].  The
+    // table is read two slabs ahead, so that the copies of the next slab start at once.
+    auto sweep = [&](auto cells) {
+        SlabBox cur{}, next{};
+        if (first_slab < nslabs) {
+            cur = slab_box(sh.box, first_slab);
+            next = slab_box(sh.box, min(first_slab + 1, nslabs - 1));
+            fetch(first_slab, cur.src);
+        }
+        __builtin_amdgcn_s_waitcnt(0);  // the direct LDS loads have landed
+        __syncthreads();
+        for (int s = first_slab; s < nslabs; ++s) {
+            if (s + 1 < nslabs) fetch(s + 1, next.src);
+            cells(s, cur, (unsigned)((s & 1) * kSlabCap));
+            cur = next;
+            next = slab_box(sh.box, min(s + 2, nslabs - 1));
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+        }
+    };
+    auto store = [&](double value) {
+        if (active) out[(long long)w.pad[0] * sview + (long long)u * su + (long long)v * sv] = (float)value;
+    };
+
+    // ---- the lane's ray (FP64 set-up) and its walk ----
+    const double pv = (double)(nV - 1 - v);  // detector row flip, Siddon_projection.cu:141
+    double sp[3];
+    ray_source(w, u, pv, sp);
+    double rx = ray_dir(w, u, pv, 0);
+    double ry = ray_dir(w, u, pv, 1);
+    double rz = ray_dir(w, u, pv, 2);
+    if (kMode == 0) {
+        // The plane walk, unless a ray of the 16 x 16 pixels around this unit has a slope of 1 or more in
+        // its view (their corner rays hold the extremes: the slopes are linear-fractional in the pixel).
+        // This depends on the pixel and the view alone, so a ray's sum does not depend on the group.
+        bool steep;
+        {
+            const int cu = min((u & ~15) + ((lane & 1) ? 15 : 0), nU - 1);
+            const double cv = (double)(nV - 1 - min((v & ~15) + ((lane & 2) ? 15 : 0), nV - 1));
+            const double dP = 0.999 * fabs(ray_dir(w, cu, cv, kP));
+            steep = __ballot(!(fabs(ray_dir(w, cu, cv, 1 - kP)) < dP && fabs(ray_dir(w, cu, cv, 2)) < dP)) != 0;
+        }
+        if (w.pad[1] != 0.0) parallel_siddon_height(sp, rx, ry, rz, nx, ny);
+        // components below 1e-3 voxel are treated as exactly zero (:155-159)
+        if (fabs(rx) < 1e-3) rx = 0.0;
+        if (fabs(ry) < 1e-3) ry = 0.0;
+        if (fabs(rz) < 1e-3) rz = 0.0;
+        const double len = sqrt(rx * rx * dvx * dvx + ry * ry * dvy * dvy + rz * rz * dvz * dvz);  // mm (:241, :267)
+        if (!steep) {  // uniform per wavefront; both branches pass the same barriers
+            const double rp = kP == 0 ? rx : ry;
+            const double da = 1.0 / fabs(rp), a0 = ((dir > 0 ? -1.0 : (double)nP + 1.0) - sp[kP]) / rp;
+            PlaneRay r;
+            r.sum = 0.0f;
+            plane_axis(sp[1 - kP], kP == 0 ? ry : rx, a0, da, nA, r.A0, r.kA, r.iA, r.dA);
+            plane_axis(sp[2], rz, a0, da, nz, r.z0, r.kz, r.iz, r.dZ);
+            if (!staged) {
+                // the beam's box does not fit an LDS buffer: read the staging copy
+                r.off = plane_offset(r, 0, 0, 0, sg.NA, nA, nz) + (unsigned)stage_index(sg, dir > 0 ? -1 : nP, 0, 0);
+                r.dZ *= sg.NA;
+                if (active)
+                    for (int c = 0; c < nP + 2; c += 8)
+                        plane_cells<false, 0, true>(r, stage, 0u, (unsigned)(dir * sg.NZ * sg.NA), nA, nz, c,
+                                                    min(8, nP + 2 - c));
+            } else {
+                r.dZ *= na;
+                int at0 = 0;         // origin offset of the box that r.off refers to
+                bool carry = false;  // r.off is the ray's voxel
+                sweep([&](int s, const SlabBox& box, unsigned at) {
+                    const int first = planes * s, count = min(planes, cells_total - first);
+                    const bool was = carry;
+                    bool rim = box.z0 != 0;
+                    if (rim || count < 8) {
+                        // what matters is whether this wavefront's rays leave the volume
+                        const int e = plane_range(r, first, count, nA, nz);
+                        const bool out = __ballot(active && e != 0) == 0;  // all stay outside: nothing to add
+                        rim = __ballot(active && e != 2) != 0;
+                        carry = false;
+                        if (out) return;
+                    }
+                    if (was)
+                        r.off -= (unsigned)(box.a0 - at0);  // from box to box by a uniform shift
+                    else
+                        r.off = plane_offset(r, first, box.a0, 0, na, nA, nz);
+                    carry = !rim && count == 8;
+                    at0 = box.a0;
+                    if (!active) return;
+                    if (count < 8)
+                        plane_cells<true, 0, true>(r, sh.buf, at, (unsigned)SP, nA, nz, first, count);
+                    else if (rim)
+                        plane_cells<true, kPlaneStride, true>(r, sh.buf, at, 0u, nA, nz, first, 8);
+                    else
+                        plane_cells<true, kPlaneStride, false>(r, sh.buf, at, 0u, nA, nz, first, 8);
+                });
+            }
+            store((double)r.sum * (len * da));  // the sum is in cells
+            return;
+        }
+        RayWalk r;
+        r.sum = 0.0f;
+        int state = 0;  // 0: no ray or finished, 1: waiting for the slab of its entry, 2: walking
+        int ip0 = 0, ia0 = 0, iz0 = 0, sx = 0, sy = 0, sz = 0;
+        double am = -INFINITY, aM = INFINITY;
+        bool hit = active && slab(sp[0], rx, nx, am, aM);
+        hit = hit && slab(sp[1], ry, ny, am, aM);
+        hit = hit && slab(sp[2], rz, nz, am, aM);
+        if (hit && am < aM) {  // a ray that misses the volume projects to 0 (:179-180)
+            const Axis ax = axis_setup(sp[0], rx, am);
+            const Axis ay = axis_setup(sp[1], ry, am);
+            const Axis az = axis_setup(sp[2], rz, am);
+            r.tx = r.t0x = ax.t0;
+            r.ty = r.t0y = ay.t0;
+            r.tz = r.t0z = az.t0;
+            r.dtx = ax.dt;
+            r.dty = ay.dt;
+            r.dtz = az.dt;
+            r.kx = r.ky = r.kz = 0.0f;
+            r.T = (float)(aM - am);
+            r.tc = 0.0f;
+            ip0 = kP == 0 ? ax.idx : ay.idx;
+            ia0 = kP == 0 ? ay.idx : ax.idx;
+            iz0 = az.idx;
+            sx = ax.step;
+            sy = ay.step;
+            sz = az.step;
+            state = 1;
+        }
+        if (!staged) {
             if (state == 1) {
                 r.off = (unsigned)stage_index(sg, ip0, iz0, ia0);
                 r.dX = (unsigned)(sx * (kP == 0 ? sg.NZ * sg.NA : 1));
@@ -517,115 +753,126 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
                 r.kexit = -1;  // never reached
                 walk<kP, false>(r, stage, 0u, (nx + ny + nz + 10) / 4);
             }
-        } else if (state == 2) {
-            // box origin (-1, -1, -4): the bordered staging copy itself
-            sample_slab<kMode, false>(rs, stage, 0u, sg.NZ * sg.NA, sg.NA, -1, -1, -4, -1, last_cell, dir,
-                                      (float)nP, (float)nA, (float)nz);
-        }
-    } else {
-        const int SP = nzb * na;
-        const int splanes = planes + tap;  // staged planes per slab
-        if (kMode == 0) {
+        } else {
             // offset steps inside a box
-            r.dX = (unsigned)(sx * (kP == 0 ? SP : 1));
-            r.dY = (unsigned)(sy * (kP == 1 ? SP : 1));
+            r.dX = (unsigned)(kP == 0 ? SP : sx);
+            r.dY = (unsigned)(kP == 1 ? SP : sy);
             r.dZ = (unsigned)(sz * na);
-        }
-        // this thread's quads of a box: row (plane * nzb + z) and 4-float column
-        const int nq4 = na >> 2, nq = splanes * nzb * nq4;
-        unsigned long long qoff[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int q = min(tid + j * kBeamThreads, nq - 1);
-            const int row = q / nq4, aq = q - row * nq4;
-            const int pl = row / nzb, zr = row - pl * nzb;
-            qoff[j] = ((unsigned long long)pl * (unsigned)sg.NZ + (unsigned)zr) * (unsigned)sg.NA + 4u * aq;
-        }
-        const int wave_first = tid & ~63;
-        // Direct global-to-LDS copies (16 bytes per lane) of slab s: quad q lands
-        // at buf[4 q]; the LDS base of each instruction is uniform per wavefront.
-        auto fetch = [&](int s, float* dst) {
-            int lo, hi;
-            slab_range(s, planes, dir, last_cell, lo, hi);
-            const int2 o = sh.origin[s];
-            const unsigned long long base = stage_index(sg, lo, o.y, o.x);
-            const int nqs = (hi - lo + 1 + tap) * nzb * nq4;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                if (wave_first + j * kBeamThreads < nqs) {
-                    if (tid + j * kBeamThreads < nqs)
-                        __builtin_amdgcn_global_load_lds(stage + base + qoff[j], dst + 4 * (wave_first + j * kBeamThreads),
-                                                         16, 0, 0);
-                }
-            }
-        };
-        fetch(0, sh.buf);
-        __builtin_amdgcn_s_waitcnt(0);  // the direct LDS loads have landed
-        __syncthreads();
-        int plo = 0, pa0 = 0, pz0 = 0;
-        for (int s = 0; s < nslabs; ++s) {
-            if (s + 1 < nslabs) fetch(s + 1, sh.buf + ((s + 1) & 1) * kSlabCap);
-            int lo, hi;
-            slab_range(s, planes, dir, last_cell, lo, hi);
-            const int2 o = sh.origin[s];
-            const unsigned slot = (unsigned)((s & 1) * kSlabCap);
-            if (kMode == 0) {
+            int at0 = 0;
+            sweep([&](int s, const SlabBox& box, unsigned at) {
+                int lo, hi;
+                slab_range(s, planes, dir, last_cell, lo, hi);
                 if (state == 2) {
                     // paused at the first plane of this slab: re-base the offset
-                    r.off += (unsigned)(-((lo - plo) * SP + (o.y - pz0) * na + (o.x - pa0)));
+                    r.off -= (unsigned)(planes * SP + box.a0 - at0);
                     r.kexit += planes;
                 } else if (state == 1 && ip0 >= lo && ip0 <= hi) {
-                    r.off = (unsigned)(((ip0 - lo) * nzb + (iz0 - o.y)) * na + (ia0 - o.x));
-                    r.kexit = dir > 0 ? hi + 1 - ip0 : ip0 - lo + 1;
+                    const int pl = dir > 0 ? ip0 - lo : hi - ip0;
+                    r.off = (unsigned)(pl * SP + iz0 * na + ia0 - box.a0);
+                    r.kexit = hi - lo + 1 - pl;
                     state = 2;
                 }
                 if (state == 2) {
                     // crossings inside one slab: its planes plus the box's a and z planes
-                    if (walk<kP, true>(r, sh.buf, slot, (planes + na + nzb + 7) / 4)) state = 0;
+                    if (walk<kP, true>(r, sh.buf, at, (planes + na + nzb + 7) / 4)) state = 0;
                 }
-            } else if (state == 2) {
-                if (sample_slab<kMode, true>(rs, sh.buf, slot, SP, na, lo, o.y, o.x, lo, hi, dir, (float)nP,
-                                             (float)nA, (float)nz))
-                    state = 0;
-            }
-            plo = lo;
-            pa0 = o.x;
-            pz0 = o.y;
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
+                at0 = box.a0;
+            });
         }
-    }
-
-    if (active) {
-        float* dst = out + (long long)w.pad[0] * sview + (long long)u * su + (long long)v * sv;
-        *dst = (float)((double)(kMode == 0 ? r.sum : rs.sum) * len);
+        store((double)r.sum * len);
+    } else {
+        RaySamples rs;
+        rs.sum = 0.0f;
+        bool on = false;
+        double len = 0.0;
+        // samples per ray and step (ray_interpolated_projection.cu:164-169)
+        const double n = sample_count(w, sqrt(rx * rx + ry * ry + rz * rz), acc);
+        if (active && n >= 1.0 && n < 1e9) {  // else: degenerate ray (pixel at the source), 0
+            const double st[3] = {rx / n, ry / n, rz / n};
+            // sample range [first, last] of the reference (:182-193), clipped to
+            // the samples strictly inside (-1, n) on every axis (the others are
+            // exactly zero)
+            const double last = (w.cap < n) ? ceil(w.cap) : n;
+            double lo = -INFINITY, hi = INFINITY;
+            const int nn[3] = {nx, ny, nz};
+            bool empty = false;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                if (st[a] == 0.0) {
+                    if (!(sp[a] > -1.0 && sp[a] < (double)nn[a])) empty = true;
+                } else {
+                    const double a0 = (-1.0 - sp[a]) / st[a], a1 = ((double)nn[a] - sp[a]) / st[a];
+                    lo = fmax(lo, fmin(a0, a1));
+                    hi = fmin(hi, fmax(a0, a1));
+                }
+            }
+            const double i0 = fmax(w.first, floor(lo));
+            const double i1 = fmin(last, ceil(hi));
+            len = sqrt(st[0] * dvx * st[0] * dvx + st[1] * dvy * st[1] * dvy + st[2] * dvz * st[2] * dvz);
+            if (!empty && i0 <= i1) {
+                // positions relative to the first sample keep the FP32 loop accurate
+                rs.qP = (float)(sp[kP] + i0 * st[kP]);
+                rs.qA = (float)(sp[1 - kP] + i0 * st[1 - kP]);
+                rs.qz = (float)(sp[2] + i0 * st[2]);
+                rs.fP = (float)st[kP];
+                rs.fA = (float)st[1 - kP];
+                rs.fz = (float)st[2];
+                rs.m = 0;
+                rs.count = (int)(i1 - i0) + 1;
+                on = true;
+            }
+        }
+        if (!staged) {
+            // box origin (-1, -1, -4): the bordered staging copy itself
+            if (on)
+                sample_slab<kMode, false>(rs, stage, 0u, sg.NZ * sg.NA, sg.NA, -1, -1, -4, -1, last_cell, dir,
+                                          (float)nP, (float)nA, (float)nz);
+        } else {
+            sweep([&](int s, const SlabBox& box, unsigned at) {
+                int lo, hi;
+                slab_range(s, planes, dir, last_cell, lo, hi);
+                if (on && sample_slab<kMode, true>(rs, sh.buf, at, SP, na, lo, box.z0, box.a0, lo, hi, dir, (float)nP,
+                                                   (float)nA, (float)nz))
+                    on = false;
+            });
+        }
+        store((double)rs.sum * len);
     }
 }
 
-// Workgroup L of one projection: tile L % tiles of group L / tiles (stacked
-// by two: tiles of 2 x 1 detector tiles; by four: 2 x 2).
+// Logical block of hardware block b: runs of kRun consecutive ones on each XCD (blocks are dealt round-robin to
+// the eight XCDs), all XCDs near the same place.
+__device__ __forceinline__ int beam_logical_block(int b, int nblk) {
+    constexpr int kRun = 64;
+    const int seg = b / (8 * kRun), r = b - seg * 8 * kRun;
+    return (seg + 1) * 8 * kRun <= nblk ? seg * 8 * kRun + (r & 7) * kRun + (r >> 3) : b;
+}
+
+// Workgroup L of one projection: tile rows slowest, then the groups, then the tiles of a row, so that the
+// launch works through the volume in bands of z, which stay in the Infinity Cache over the groups (512^3,
+// 360 views: 30.5 ms against 32.4 with the groups slowest).
 template <int kMode>
 __device__ __forceinline__ void beam_block(const float* __restrict__ stage_x, const float* __restrict__ stage_y,
                                            int nx, int ny, int nz, int na_x, int na_y,
                                            const FwdView* __restrict__ views, const BeamGroup* __restrict__ groups,
                                            int ngroups, int nU, int nV, long long su, long long sv, long long sview,
                                            float* __restrict__ out, double acc, double dvx, double dvy, double dvz,
-                                           int max_planes, int stack, int L, SweepShared& sh) {
-    const int edge_u = stack >= 2 ? 2 * kBeamTile : kBeamTile, edge_v = stack == 4 ? 2 * kBeamTile : kBeamTile;
+                                           int max_planes, BeamShape shape, int L, SweepShared& sh) {
+    const int edge_u = 16 * shape.units_u, edge_v = 4 * shape.units_v;
     const int tilesU = (nU + edge_u - 1) / edge_u, tilesV = (nV + edge_v - 1) / edge_v;
-    const int tiles = tilesU * tilesV;
-    const int gi = L / tiles, tile = L % tiles;
-    if (gi >= ngroups) return;  // uniform per workgroup
+    const int row = ngroups * tilesU;
+    const int tile_v = L / row, gi = (L - tile_v * row) / tilesU, tile_u = L - tile_v * row - gi * tilesU;
+    if (tile_v >= tilesV) return;  // uniform per workgroup
     const BeamGroup grp = groups[gi];
     StageGeom sg;
     sg.NZ = nz + 2;
     if (grp.principal == 0) {
         sg.NA = na_x + 8;
-        beam_sweep<0, kMode>(stage_x, sg, nx, ny, nz, views, grp, tile % tilesU, tile / tilesU, stack, nU, nV, su, sv,
+        beam_sweep<0, kMode>(stage_x, sg, nx, ny, nz, views, grp, tile_u, tile_v, shape, nU, nV, su, sv,
                              sview, out, acc, dvx, dvy, dvz, max_planes, sh);
     } else {
         sg.NA = na_y + 8;
-        beam_sweep<1, kMode>(stage_y, sg, nx, ny, nz, views, grp, tile % tilesU, tile / tilesU, stack, nU, nV, su, sv,
+        beam_sweep<1, kMode>(stage_y, sg, nx, ny, nz, views, grp, tile_u, tile_v, shape, nU, nV, su, sv,
                              sview, out, acc, dvx, dvy, dvz, max_planes, sh);
     }
 }
@@ -637,10 +884,10 @@ __global__ __launch_bounds__(kBeamThreads) __attribute__((amdgpu_waves_per_eu(8,
     const float* __restrict__ stage_x, const float* __restrict__ stage_y, int nx, int ny, int nz, int na_x, int na_y,
     const FwdView* __restrict__ views, const BeamGroup* __restrict__ groups, int ngroups, int nU, int nV,
     long long su, long long sv, long long sview, float* __restrict__ out, double acc, double dvx, double dvy,
-    double dvz, int max_planes, int stack) {
+    double dvz, int max_planes, BeamShape shape) {
     __shared__ SweepShared sh;
     beam_block<kMode>(stage_x, stage_y, nx, ny, nz, na_x, na_y, views, groups, ngroups, nU, nV, su, sv, sview, out,
-                      acc, dvx, dvy, dvz, max_planes, stack, xcd_logical_block(blockIdx.x, gridDim.x), sh);
+                      acc, dvx, dvy, dvz, max_planes, shape, beam_logical_block(blockIdx.x, gridDim.x), sh);
 }
 
 // Siddon projections of many independent problems (Python detector layout) in
@@ -649,12 +896,12 @@ __global__ __launch_bounds__(kBeamThreads) __attribute__((amdgpu_waves_per_eu(8,
 __global__ __launch_bounds__(kBeamThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void ax_beam_multi_kernel(
     const BeamJob* __restrict__ jobs, int njobs) {
     __shared__ SweepShared sh;
-    const int L = xcd_logical_block(blockIdx.x, gridDim.x);
+    const int L = beam_logical_block(blockIdx.x, gridDim.x);
     const int j = find_job(jobs, njobs, L);
     const BeamJob& J = jobs[j];
     beam_block<0>(J.stage_x, J.stage_y, J.nx, J.ny, J.nz, J.na_x, J.na_y, J.views,
                   reinterpret_cast<const BeamGroup*>(J.groups), J.ngroups, J.nU, J.nV, 1, J.nU,
-                  (long long)J.nU * J.nV, J.out, J.acc, J.dvx, J.dvy, J.dvz, J.max_planes, J.stack, L - J.begin, sh);
+                  (long long)J.nU * J.nV, J.out, J.acc, J.dvx, J.dvy, J.dvz, J.max_planes, J.shape, L - J.begin, sh);
 }
 
 // Staging copy for principal axis P: out[p][z][a] over the bordered ranges
@@ -732,9 +979,9 @@ int stage_job_blocks(const HostGeometry& g, int principal, int* gx, int* gy) {
     return *gx * *gy * (g.nVoxel[2] + 2);
 }
 
-long long beam_job_blocks(const HostGeometry& g, int ngroups, int stack) {
-    const int edge_u = stack >= 2 ? 2 * kBeamTile : kBeamTile, edge_v = stack == 4 ? 2 * kBeamTile : kBeamTile;
-    const long long tiles = ((g.nDetec[0] + edge_u - 1) / edge_u) * ((g.nDetec[1] + edge_v - 1) / edge_v);
+long long beam_job_blocks(const HostGeometry& g, int ngroups, const BeamShape& shape) {
+    const int edge_u = 16 * shape.units_u, edge_v = 4 * shape.units_v;
+    const long long tiles = (long long)((g.nDetec[0] + edge_u - 1) / edge_u) * ((g.nDetec[1] + edge_v - 1) / edge_v);
     return tiles * ngroups;
 }
 
@@ -770,7 +1017,7 @@ int launch_stage_volume(const void* vol, int dtype, const HostGeometry& g, int p
 }
 
 int launch_ax_beam(const float* stage_x, const float* stage_y, const HostGeometry& g, const FwdView* d_views,
-                   const int* d_groups, int ngroups, int stack, int projection_type, int layout, float* proj,
+                   const int* d_groups, int ngroups, const BeamShape& shape, int projection_type, int layout, float* proj,
                    int max_planes, hipStream_t stream) {
     TIGRE_REQUIRE(max_planes >= 1 && max_planes <= kSlabPlanesMax, "slab planes out of range");
     const long long nU = g.nDetec[0], nV = g.nDetec[1];
@@ -779,7 +1026,7 @@ int launch_ax_beam(const float* stage_x, const float* stage_y, const HostGeometr
         su = nV;
         sv = 1;
     }
-    const long long blocks = beam_job_blocks(g, ngroups, stack);
+    const long long blocks = beam_job_blocks(g, ngroups, shape);
     TIGRE_REQUIRE(blocks < (1LL << 31), "too many detector tiles for one launch");
     // LDS offsets are 32-bit; global element offsets of the staging copy too
     TIGRE_REQUIRE(stage_elements(g, 0) < (1LL << 32) && stage_elements(g, 1) < (1LL << 32),
@@ -791,7 +1038,7 @@ int launch_ax_beam(const float* stage_x, const float* stage_y, const HostGeometr
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBeamThreads), 0, stream, stage_x, stage_y, g.nVoxel[0],
                        g.nVoxel[1], g.nVoxel[2], stage_pad(g.nVoxel[1]), stage_pad(g.nVoxel[0]), d_views,
                        reinterpret_cast<const BeamGroup*>(d_groups), ngroups, g.nDetec[0], g.nDetec[1], su, sv,
-                       nU * nV, proj, g.accuracy, g.dVoxel[0], g.dVoxel[1], g.dVoxel[2], max_planes, stack);
+                       nU * nV, proj, g.accuracy, g.dVoxel[0], g.dVoxel[1], g.dVoxel[2], max_planes, shape);
     TIGRE_HIP_TRY(hipGetLastError());
     return TIGRE_OK;
 }

@@ -218,12 +218,15 @@ int launch_ax_siddon(const float* bricked, const HostGeometry& g, const BrickGri
 long long stage_elements(const HostGeometry& g, int principal);
 int launch_stage_volume(const void* vol, int dtype, const HostGeometry& g, int principal, float* stage,
                         hipStream_t stream);
+// The rays of a beam workgroup: a tile of units_u x units_v units of 16 x 4 pixels in each of
+// 16 / (units_u units_v) views.
+struct BeamShape {
+    int units_u, units_v;
+};
 // Beam-staged forward projection (Siddon or interpolated); d_groups: ngroups
-// records {first view, view count (1..4), principal, direction}; stack: the
-// detector tiles a workgroup traces per view (1; 2 when no group holds more
-// than two views; 4, as 2 x 2, when every group holds one).
+// records {first view, view count (1..4), principal, direction}.
 int launch_ax_beam(const float* stage_x, const float* stage_y, const HostGeometry& g, const FwdView* d_views,
-                   const int* d_groups, int ngroups, int stack, int projection_type, int layout, float* proj,
+                   const int* d_groups, int ngroups, const BeamShape& shape, int projection_type, int layout, float* proj,
                    int max_planes, hipStream_t stream);
 int launch_ax_interp(const float* bricked, const HostGeometry& g, const BrickGrid& b, const FwdView* d_views,
                      int nviews, int layout, float* proj, hipStream_t stream);
@@ -256,7 +259,7 @@ struct ForwardRecords {
     std::vector<int> groups;
     int nbeam = 0;
     bool stage_used[2] = {false, false};
-    int stack = 1;  // detector tiles per view of a beam workgroup: 1, 2 or 4
+    BeamShape shape{1, 4};
     int ngroups() const { return (int)groups.size() / 4; }
     int nrest() const { return (int)ordered.size() - nbeam; }
 };
@@ -294,7 +297,8 @@ struct BeamJob {     // beam-staged Siddon projection of one view list
     const int* groups;
     float* out;
     double acc, dvx, dvy, dvz;
-    int nx, ny, nz, na_x, na_y, ngroups, nU, nV, max_planes, begin, stack;
+    int nx, ny, nz, na_x, na_y, ngroups, nU, nV, max_planes, begin;
+    BeamShape shape;
 };
 struct ResidualJob { // r = W (p - Ax), n elements
     const float* proj;
@@ -340,7 +344,7 @@ int launch_quad_multi(const QuadJob* d_jobs, int njobs, long long blocks, hipStr
 int launch_atb_multi(const AtbJob* d_jobs, int njobs, long long blocks, int zper, hipStream_t stream);
 // Block counts of one job of each kind (host side).
 int stage_job_blocks(const HostGeometry& g, int principal, int* gx, int* gy);
-long long beam_job_blocks(const HostGeometry& g, int ngroups, int stack);
+long long beam_job_blocks(const HostGeometry& g, int ngroups, const BeamShape& shape);
 int residual_job_blocks(long long n);
 int quad_job_blocks(int nU, int nV, int nviews);
 

@@ -115,19 +115,21 @@ void build_forward_records(const HostGeometry& g, bool interp, int views_per_gro
     rec->nbeam = (int)rec->ordered.size();
     for (int i : rest) rec->ordered.push_back(views[i]);
     // Groups of fewer than four views leave view slots of a workgroup empty:
-    // when no group holds more than two views, every workgroup traces two
-    // tiles of each of its views, and when every group holds one view, 2 x 2
-    // tiles of it, provided the launch keeps a workgroup for every CU of the
-    // 256-CU MI355X (a single view of a 256 x 256 detector stacked into 64
-    // workgroups measured 0.116 against 0.058 ms unstacked; of a 512 x 512
-    // one, into 256, 0.221 against 0.250 ms).
+    // when no group holds more than two views, every workgroup traces twice the
+    // pixels of each of its views, and when every group holds one view, four times,
+    // provided the launch keeps a workgroup for every CU of the 256-CU MI355X (a
+    // single view of a 256 x 256 detector in 64 workgroups measured 0.116 against
+    // 0.058 ms in 16 x 16 tiles; of a 512 x 512 one, in 256, 0.221 against 0.250 ms).
+    // Siddon's tiles are wide along u: the box of a 32 x 8 tile in four views has fewer rows than that of a
+    // 16 x 16 one, and longer ones, which waste less of their 128-byte lines (512^3, 360 views 25.3 against
+    // 26.4 ms; a ragged 200^3 volume with 4-degree spacing, whose 16 x 16 boxes do not fit eight planes, 0.68
+    // against 0.74 ms; one view a group, 64 x 16 against 32 x 32: 512^3, 20 views 3.13 against 3.34 ms).
     int most = 0;
     for (int k = 0; k < rec->ngroups(); ++k) most = std::max(most, rec->groups[4 * k + 1]);
-    rec->stack = 1;
+    rec->shape = interp ? BeamShape{1, 4} : BeamShape{2, 2};
     if (most == 1 || most == 2) {
-        const int st = most == 1 ? 4 : 2, edge_v = st == 4 ? 32 : 16;
-        const long long tiles = (long long)((g.nDetec[0] + 31) / 32) * ((g.nDetec[1] + edge_v - 1) / edge_v);
-        if (tiles * rec->ngroups() >= 256) rec->stack = st;
+        const BeamShape more = most == 2 ? BeamShape{2, 4} : (interp ? BeamShape{2, 8} : BeamShape{4, 4});
+        if (beam_job_blocks(g, rec->ngroups(), more) >= 256) rec->shape = more;
     }
 }
 
@@ -158,7 +160,7 @@ int ax_launch(const void* d_img, int dtype, const HostGeometry& g, const Forward
         TIGRE_CHECK(launch_stage_volume(d_img, dtype, g, a, stage[a], stream));
     }
     if (rec.ngroups() > 0)
-        TIGRE_CHECK(launch_ax_beam(stage[0], stage[1], g, d_views, d_groups, rec.ngroups(), rec.stack,
+        TIGRE_CHECK(launch_ax_beam(stage[0], stage[1], g, d_views, d_groups, rec.ngroups(), rec.shape,
                                    projection_type, layout, d_proj, max_planes, stream));
     if (rec.nrest() > 0) {
         const BrickGrid b = interp ? interp_bricks(g) : siddon_bricks(g);

@@ -353,8 +353,8 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
             j.nV = g.nDetec[1];
             j.max_planes = p->max_planes;
             j.begin = (int)b_beam;
-            j.stack = rec.stack;
-            b_beam += beam_job_blocks(g, rec.ngroups(), rec.stack);
+            j.shape = rec.shape;
+            b_beam += beam_job_blocks(g, rec.ngroups(), rec.shape);
             beam.push_back(j);
         }
         if (rec.nrest() > 0) rest_steps.push_back(i);
