@@ -239,7 +239,10 @@ struct AtbUpdate {
     const float* inv_v = nullptr;
     int noneg = 0;
 };
-// zper: slices per lane, 4, 8 or 16.
+// zper: slices per lane, 4, 8 or 16; 16 lets axial views take what suits the volume.
+// Slices per lane that an axial backprojection takes for the requested zper, alone or in a batch; 4, 8 and 16 give
+// the same bits, and 32 is taken in both or in neither.
+int staged_slices(const HostGeometry& g, int zper, bool batched);
 int launch_atb(const float* quads, const HostGeometry& g, const BwdView* d_views, bool matched,
                bool axial, float* vol, int zper, const AtbUpdate& ep, hipStream_t stream);
 int run_pocs_tv(const float* img, float* dst, float alpha, long nx, long ny, long nz, int maxiter,
@@ -383,9 +386,10 @@ int launch_store_converted(const float* src, void* dst, long long n, int dtype, 
 // Quad projection dimensions: tap origins -1 .. n on each detector axis.
 __host__ __device__ inline long quad_det(int n) { return (long)n + 2; }
 // Rows of quads allocated after the last view of a quad copy: the staged
-// backprojector copies whole 4 x 16-quad blocks of a detector window, which
-// may run up to 23 rows past a view's last row and 15 quads past a row's end
-// (into the next view or row, never read; past the last view, into this slack).
+// backprojector copies whole 2 x 32-quad blocks of a detector window, which may
+// run one row past a view's last row and 31 quads past a row's end, eleven rows
+// of the narrowest detector (into the next view or row, never read; past the
+// last view, into this slack).
 constexpr long kQuadSlackRows = 25;
 
 }  // namespace tigre

@@ -77,9 +77,9 @@ struct TigreBatch_ {
     const BeamJob* d_beam = nullptr;
     const ResidualJob* d_res = nullptr;
     const QuadJob* d_quad = nullptr;
-    const AtbJob* d_atb[3] = {nullptr, nullptr, nullptr};  // slices per lane 4, 8, 16
-    int n_stage = 0, n_beam = 0, n_res = 0, n_quad = 0, n_atb[3] = {0, 0, 0};
-    long long b_stage = 0, b_beam = 0, b_res = 0, b_quad = 0, b_atb[3] = {0, 0, 0};
+    const AtbJob* d_atb[4] = {nullptr, nullptr, nullptr, nullptr};  // slices per lane 4, 8, 16, 32
+    int n_stage = 0, n_beam = 0, n_res = 0, n_quad = 0, n_atb[4] = {0, 0, 0, 0};
+    long long b_stage = 0, b_beam = 0, b_res = 0, b_quad = 0, b_atb[4] = {0, 0, 0, 0};
     std::vector<TigreBatchStep> steps;
     std::vector<int> rest_steps;  // steps with views for the gather kernels
     std::vector<int> atb_steps;   // steps whose backprojection runs on its own
@@ -90,7 +90,7 @@ struct TigreBatch_ {
 
 namespace {
 
-int zslot(int zper) { return zper == 4 ? 0 : (zper == 8 ? 1 : 2); }
+int zslot(int zper) { return zper == 4 ? 0 : zper == 8 ? 1 : zper == 16 ? 2 : 3; }
 
 // Byte offset of the staging copy for principal axis a in a forward workspace
 // (the layout ax_launch uses), and of the bricked copy after them.
@@ -102,8 +102,8 @@ size_t stage_offset(const HostGeometry& g, const ForwardRecords& rec, int a) {
 }
 
 bool atb_multi_ok(const TigrePlan_* p) {
-    // the staged kernel: FDK weight, axial views, row pairs in 16 bits
-    return p->axial && !p->g.parallel && p->g.nDetec[1] + 1 < 65536;
+    // the staged kernel with the FDK weight
+    return p->axial && !p->g.parallel;
 }
 
 }  // namespace
@@ -289,8 +289,8 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
     std::vector<BeamJob> beam;
     std::vector<ResidualJob> res;
     std::vector<QuadJob> quad;
-    std::vector<AtbJob> atb[3];
-    long long b_stage = 0, b_beam = 0, b_res = 0, b_quad = 0, b_atb[3] = {0, 0, 0};
+    std::vector<AtbJob> atb[4];
+    long long b_stage = 0, b_beam = 0, b_res = 0, b_quad = 0, b_atb[4] = {0, 0, 0, 0};
     std::vector<int> rest_steps, atb_steps;
     std::vector<const void*> owned;  // buffers a step writes: no two steps may share one
     for (int i = 0; i < nsteps; ++i) {
@@ -387,7 +387,7 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
                           quad_det(g.nDetec[0]) * quad_det(g.nDetec[1]) * 16 < (1LL << 32),
                       "detector too large for one backprojection launch");
         if (atb_multi_ok(p)) {
-            const int k = zslot(p->zper);
+            const int z = staged_slices(g, p->zper, true), k = zslot(z);
             AtbJob j;
             j.quads = reinterpret_cast<const float*>(ws);
             j.views = static_cast<const BwdView*>(p->d_bwd);
@@ -404,7 +404,7 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
             j.noneg = st.noneg ? 1 : 0;
             j.gx = (j.nx + 15) / 16;
             j.gy = (j.ny + 15) / 16;
-            const int gz = (j.nz + p->zper - 1) / p->zper;
+            const int gz = (j.nz + z - 1) / z;
             TIGRE_REQUIRE(j.gy <= 65535 && gz <= 65535, "volume too large for one launch");
             j.begin = (int)b_atb[k];
             b_atb[k] += (long long)j.gx * j.gy * gz;
@@ -414,7 +414,8 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
         }
     }
     TIGRE_REQUIRE(b_stage < (1LL << 31) && b_beam < (1LL << 31) && b_res < (1LL << 31) && b_quad < (1LL << 31) &&
-                      b_atb[0] < (1LL << 31) && b_atb[1] < (1LL << 31) && b_atb[2] < (1LL << 31),
+                      b_atb[0] < (1LL << 31) && b_atb[1] < (1LL << 31) && b_atb[2] < (1LL << 31) &&
+                      b_atb[3] < (1LL << 31),
                   "batch too large for one launch per stage");
     TigreBatch_* b = new TigreBatch_();
     int st = [&]() -> int {
@@ -423,19 +424,19 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
         b->rest_steps = rest_steps;
         b->atb_steps = atb_steps;
         // one table allocation: every array at a 256-byte boundary
-        const size_t sizes[7] = {stage.size() * sizeof(StageJob), beam.size() * sizeof(BeamJob),
+        const size_t sizes[8] = {stage.size() * sizeof(StageJob), beam.size() * sizeof(BeamJob),
                                  res.size() * sizeof(ResidualJob), quad.size() * sizeof(QuadJob),
                                  atb[0].size() * sizeof(AtbJob), atb[1].size() * sizeof(AtbJob),
-                                 atb[2].size() * sizeof(AtbJob)};
-        const void* src[7] = {stage.data(), beam.data(), res.data(), quad.data(), atb[0].data(), atb[1].data(),
-                              atb[2].data()};
-        size_t off[7], total = 0;
-        for (int k = 0; k < 7; ++k) {
+                                 atb[2].size() * sizeof(AtbJob), atb[3].size() * sizeof(AtbJob)};
+        const void* src[8] = {stage.data(), beam.data(), res.data(), quad.data(), atb[0].data(), atb[1].data(),
+                              atb[2].data(), atb[3].data()};
+        size_t off[8], total = 0;
+        for (int k = 0; k < 8; ++k) {
             off[k] = total;
             total += align256(sizes[k]);
         }
         std::vector<char> host(total, 0);
-        for (int k = 0; k < 7; ++k)
+        for (int k = 0; k < 8; ++k)
             if (sizes[k]) std::memcpy(host.data() + off[k], src[k], sizes[k]);
         TIGRE_CHECK(upload_sync(&b->d_tables, host.data(), total));
         const char* base = static_cast<const char*>(b->d_tables);
@@ -443,12 +444,12 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
         b->d_beam = reinterpret_cast<const BeamJob*>(base + off[1]);
         b->d_res = reinterpret_cast<const ResidualJob*>(base + off[2]);
         b->d_quad = reinterpret_cast<const QuadJob*>(base + off[3]);
-        for (int k = 0; k < 3; ++k) b->d_atb[k] = reinterpret_cast<const AtbJob*>(base + off[4 + k]);
+        for (int k = 0; k < 4; ++k) b->d_atb[k] = reinterpret_cast<const AtbJob*>(base + off[4 + k]);
         b->n_stage = (int)stage.size();
         b->n_beam = (int)beam.size();
         b->n_res = (int)res.size();
         b->n_quad = (int)quad.size();
-        for (int k = 0; k < 3; ++k) {
+        for (int k = 0; k < 4; ++k) {
             b->n_atb[k] = (int)atb[k].size();
             b->b_atb[k] = b_atb[k];
         }
@@ -489,8 +490,8 @@ int tigre_batch_sart(TigreBatch batch, void* stream) {
     }
     TIGRE_CHECK(launch_residual_multi(b.d_res, b.n_res, b.b_res, s));
     TIGRE_CHECK(launch_quad_multi(b.d_quad, b.n_quad, b.b_quad, s));
-    const int zpers[3] = {4, 8, 16};
-    for (int k = 0; k < 3; ++k)
+    const int zpers[4] = {4, 8, 16, 32};
+    for (int k = 0; k < 4; ++k)
         if (b.n_atb[k]) TIGRE_CHECK(launch_atb_multi(b.d_atb[k], b.n_atb[k], b.b_atb[k], zpers[k], s));
     for (int i : b.atb_steps) {  // backprojections outside the staged multi-job kernel
         const TigreBatchStep& st = b.steps[i];
