@@ -166,6 +166,13 @@ int tigre_ax_parallel_device(const void* d_img, const TigreGeometry* geo, void* 
 int tigre_atb_parallel_device(const void* d_proj, const TigreGeometry* geo, void* d_vol,
                               const float* angles, int nangles, int layout, int dtype, void* stream);
 
+/* Convolves `rows` rows of nU pixels with a symmetric kernel, given by its real
+ * spectrum over 2^log2_len elements (d_response, 2^(log2_len - 1) + 1 values,
+ * scaled by 2^-log2_len); 2^log2_len is 64 .. 4096 and at least 2 nU.  With
+ * d_weight (an nV x nU image) row r is first weighted by its row r % nV. */
+int tigre_filter_rows_device(const float* d_rows, const float* d_weight, const float* d_response,
+                             float* d_out, long long rows, int nV, int nU, int log2_len, void* stream);
+
 /* maxIter TV steepest-descent steps on a device volume (X fastest); d_dst may
  * equal d_img.  image_size = {X, Y, Z}. */
 int tigre_pocs_tv_device(const float* d_img, float* d_dst, float alpha, const long* image_size,

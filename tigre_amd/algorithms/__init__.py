@@ -25,7 +25,7 @@ import numpy as np
 from .. import _native
 from ..geometry import prepared
 from ..operators import _stream_handle
-from ..utilities.filtering import filtering
+from ..utilities.filtering import filtering, weighted_filtering
 from ..utilities.order_subsets import order_subsets
 
 __all__ = ["fdk", "FDK", "fbp", "ossart", "iterativereconalg", "sart", "sirt", "sart_tv", "ossart_tv", "fista", "ista", "cgls", "lsqr",
@@ -213,7 +213,7 @@ def fdk(proj, geo, angles, filter=None, verbose=False, return_tensor=False, **kw
     yv = (np.arange(nV) - nV / 2 + 0.5) * dV
     xx, yy = np.meshgrid(xv, yv)
     w = torch.as_tensor((DSD0 / np.sqrt(DSD0 ** 2 + xx ** 2 + yy ** 2)).astype(np.float32), device=p.device)
-    filt = filtering(p * w, g, g.angles, parker=False, verbose=verbose)
+    filt = weighted_filtering(p, w, g, g.angles)
     vs = ViewSets(g, g.angles, [np.arange(len(g.angles))])
     return _result(vs.atb(filt, 0, _native.BACKPROJ_FDK), return_tensor)
 

@@ -243,6 +243,13 @@ int tigre_atb_parallel_device(const void* d_proj, const TigreGeometry* geo, void
     return atb_device(d_proj, g, d_vol, TIGRE_BACKPROJ_FDK, layout, dtype, (hipStream_t)stream);
 }
 
+int tigre_filter_rows_device(const float* d_rows, const float* d_weight, const float* d_response, float* d_out,
+                             long long rows, int nV, int nU, int log2_len, void* stream) {
+    set_error("");
+    TIGRE_REQUIRE(d_rows && d_response && d_out, "null argument");
+    return launch_filter_rows(d_rows, d_weight, d_response, d_out, rows, nV, nU, log2_len, (hipStream_t)stream);
+}
+
 int tigre_pocs_tv_device(const float* d_img, float* d_dst, float alpha, const long* image_size, int maxIter,
                          void* stream) {
     set_error("");

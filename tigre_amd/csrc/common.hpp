@@ -245,6 +245,10 @@ struct AtbUpdate {
 int staged_slices(const HostGeometry& g, int zper, bool batched);
 int launch_atb(const float* quads, const HostGeometry& g, const BwdView* d_views, bool matched,
                bool axial, float* vol, int zper, const AtbUpdate& ep, hipStream_t stream);
+// Row filter (filter.hip): transforms of 2^6 .. 2^12 elements, twice the row at least.
+constexpr int kFilterMinLog = 6, kFilterMaxLog = 12;
+int launch_filter_rows(const float* in, const float* weight, const float* response, float* out, long long rows, int nV,
+                       int nU, int log2_len, hipStream_t stream);
 int run_pocs_tv(const float* img, float* dst, float alpha, long nx, long ny, long nz, int maxiter,
                 hipStream_t stream);
 int run_aw_pocs_tv(const float* img, float* dst, float alpha, float delta, long nx, long ny, long nz, int maxiter,
