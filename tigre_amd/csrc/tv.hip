@@ -8,17 +8,14 @@
 //     g(v)   = n_x(v) + n_y(v) + n_z(v) - n_x(v + x) - n_y(v + y) - n_z(v + z),
 // (w = 1 for TV, exp(-(d / delta)^2) per component for AwTV, with the fast
 // exponential as the reference's __expf), so each n is
-// computed once per voxel instead of four times.  One iteration is two passes:
-//   pass 1  g at every voxel, sum of g^2 per workgroup (FP32 per lane over
-//           its 32 voxels at most, FP64 across lanes);
-//   scale   one workgroup sums the partials in a fixed order (the same result
-//           every run) into alpha / sqrt(sum + norm_eps);
-//   pass 2  f' = f - scale * g, recomputing g from f.
-// Each pass is a 128 x 8 column tile that marches along z through a chunk of
-// planes, every lane two columns with their z neighbours in registers and
-// their x / y neighbours through LDS, so f is read from HBM about once per pass:
-// 12 bytes of traffic per voxel and iteration, no host round trip for the
-// norm.
+// computed once per voxel instead of four times.  An iteration needs the norm
+// of the whole g before it can step, f' = f - alpha / sqrt(sum g^2 + norm_eps)
+// g, and is one pass all the same: the pass that makes f' from f also sums g^2
+// of f' for the next step (FP32 over eight voxels, FP64 beyond), and the next
+// pass adds up the workgroups' sums in a fixed order at its start, every
+// wavefront for itself.  A first pass only sums, the last only steps: no host
+// round trip for the norm, maxiter + 1 launches, 8 bytes of traffic per voxel
+// and iteration.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -29,18 +26,12 @@
 namespace tigre {
 
 namespace {
-constexpr int kTY = 8, kZC = 16;            // tile rows (one wavefront each), planes per chunk
-constexpr int kTX = 128;                    // tile columns: two adjacent ones per lane
-constexpr int kAhead = 4;                   // planes of f in flight per lane
-constexpr int kTvThreads = 64 * kTY;
-// LDS planes.  f: rows -1 .. kTY, columns -1 .. kTX at index lx + 2 (an even
-// row length, so every lane's column pair is 8-byte aligned); n: rows
-// 0 .. kTY, columns 0 .. kTX (padded to an even length).
-constexpr int kFW = kTX + 4, kFH = kTY + 2;
-constexpr int kNW = kTX + 2, kNH = kTY + 1;
-constexpr int kFHalo = 2 * (kTX + 2) + 2 * kTY;  // halo entries of an f plane
-__device__ __forceinline__ int f_index(int lx, int ly) { return (ly + 1) * kFW + lx + 2; }
-__device__ __forceinline__ int n_index(int lx, int ly) { return ly * kNW + lx; }
+constexpr int kTvThreads = 256, kTvWaves = kTvThreads / 64;  // wavefronts work on tiles of their own
+constexpr int kTvColumns = 60;                               // columns of a tile, but for the volume's edges
+template <int k>
+using Int = std::integral_constant<int, k>;
+constexpr int kTvBatch = 6;                                  // rows whose chains are interleaved
+constexpr int kTvBlocks = 1024;                              // workgroups of a pass, at most
 
 struct TvParams {
     const float* prior;  // PICCS prior image
@@ -48,66 +39,84 @@ struct TvParams {
     float ratio;         // PICCS prior ratio
 };
 
-// Workgroup sum of one double per lane (wavefront shuffles, then LDS).
+// Workgroup sum of one double per lane (wavefront shuffles, then LDS), in every thread.
 __device__ inline double block_sum(double v) {
-    __shared__ double part[kTvThreads / 64];
+    __shared__ double part[kTvWaves];
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) part[wave] = v;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
     double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int i = 0; i < kTvThreads / 64; ++i) s += part[i];
-    __syncthreads();
-    return s;  // valid in thread 0
+    for (int i = 0; i < kTvWaves; ++i) s += part[i];
+    return s;
 }
 
-// Tile-relative position of f-plane halo entry e: row -1 (x0 - 1 .. x0 + kTX),
-// row kTY, then the columns x0 - 1 and x0 + kTX of rows 0 .. kTY - 1.
-__device__ __forceinline__ void f_halo_pos(int e, int& lx, int& ly) {
-    if (e < kTX + 2) {
-        lx = e - 1;
-        ly = -1;
-    } else if (e < 2 * (kTX + 2)) {
-        lx = e - (kTX + 2) - 1;
-        ly = kTY;
-    } else {
-        const int k = e - 2 * (kTX + 2);
-        lx = k < kTY ? -1 : kTX;
-        ly = k < kTY ? k : k - kTY;
-    }
+// Value of the lane before / after this one (0 in lane 0 / 63).
+__device__ __forceinline__ float lane_before(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, true));
 }
+__device__ __forceinline__ float lane_after(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xF, 0xF, true));
+}
+// An order point for the compiler: the value is formed before the branches that follow, not after them with all that
+// it is formed from kept in registers.
+__device__ __forceinline__ void formed(float& v) { asm volatile("" : "+v"(v)); }
 
-// The normalised difference field at one voxel from its value c, the value
-// below it (z - 1) and its neighbours at x - 1 and y - 1 (GD_TV.cu:104-140:
-// a missing neighbour's difference is 0).  No masks on the differences: the
-// f planes hold, at x = -1 and y = -1, copies of the edge voxels (so those
-// differences are exactly 0), and 0 in the zero slices (plane nz, and plane
-// -1 below the first); `ok` says whether n exists at all (the column lies in
-// the volume and, for PICCS, the plane too).
-template <int kKind>
-__device__ __forceinline__ void n_field(float c, float below, float cy, float cx, bool ok, bool has_below,
-                                        const TvParams& tp, float& n0, float& n1, float& n2) {
-    constexpr bool kPadZ = kKind != 2;
+// The normalised difference field at kB voxels from their values c, the values below them (z - 1) and their
+// neighbours at x - 1 and y - 1 (GD_TV.cu:104-140: a missing neighbour's difference is 0, and beyond the high edges n
+// is 0 in its axis).  No masks: beyond the edges the rows and columns hold copies of the edge voxels, so those
+// differences are exactly 0, and the zero slices (planes -1 and nz) hold 0.  z: whether PICCS has the z difference.
+// In stages over the voxels, kept apart: left to itself the compiler finishes one voxel's chain of square root,
+// reciprocal and products after the other's, and three wavefronts a SIMD do not hide that.  n: the numerator in z, the
+// field in y and x; s: what the numerator is to be multiplied with.
+template <int kKind, int kB>
+__device__ __forceinline__ void n_field(const float (&c)[kB], const float (&below)[kB], const float (&cy)[kB], bool z,
+                                        const TvParams& tp, float (&n)[kB][3], float (&s)[kB]) {
     constexpr float eps = kKind == 2 ? 1e-6f : 1e-8f;
-    // branch-free: where n does not exist the reciprocal is replaced by 0, so
-    // n is +-0 (every operand is finite: f planes hold loaded values or 0)
-    const float d0 = kPadZ ? c - below : (has_below ? c - below : 0.0f);
-    const float d1 = c - cy;
-    const float d2 = c - cx;
-    float w0 = 1.0f, w1 = 1.0f, w2 = 1.0f;
-    if (kKind == 1) {
-        const float a0 = d0 * tp.inv_delta, a1 = d1 * tp.inv_delta, a2 = d2 * tp.inv_delta;
-        w0 = __expf(-a0 * a0);
-        w1 = __expf(-a1 * a1);
-        w2 = __expf(-a2 * a2);
+    float d[kB][3], w[kB][3];
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+        d[i][0] = kKind == 2 ? (z ? c[i] - below[i] : 0.0f) : c[i] - below[i];
+        d[i][1] = c[i] - cy[i];
+        d[i][2] = c[i] - lane_before(c[i]);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kKind == 1) {
+#pragma unroll
+        for (int i = 0; i < kB; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float a = d[i][k] * tp.inv_delta;
+                w[i][k] = __expf(-a * a);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+        const float(&e)[3] = d[i];
+        if (kKind == 0) s[i] = fmaf(e[2], e[2], fmaf(e[0], e[0], e[1] * e[1]));
+        if (kKind == 1) s[i] = fmaf(e[2], w[i][2] * e[2], fmaf(e[0], w[i][0] * e[0], e[1] * (w[i][1] * e[1])));
+        if (kKind == 2) s[i] = fmaf(e[2], e[2], fmaf(e[1], e[1], e[0] * e[0]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
     // hardware square root and reciprocal (1 ulp each)
-    const float inv = __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(w0 * d0 * d0 + w1 * d1 * d1 + w2 * d2 * d2) + eps);
-    const float s = ok ? inv : 0.0f;
-    n0 = w0 * d0 * s;
-    n1 = w1 * d1 * s;
-    n2 = w2 * d2 * s;
+#pragma unroll
+    for (int i = 0; i < kB; ++i) s[i] = __builtin_amdgcn_sqrtf(s[i]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kB; ++i) s[i] = __builtin_amdgcn_rcpf(s[i] + eps);
+    __builtin_amdgcn_sched_barrier(0);
+    // rounded products: g takes an n once as a voxel's own and once as its neighbour's, and where the two should cancel
+    // they have to be the same number (what is left of them is normalised in the next iteration)
+    {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            n[i][0] = kKind == 1 ? w[i][0] * d[i][0] : d[i][0];
+#pragma unroll
+            for (int k = 1; k < 3; ++k) n[i][k] = (kKind == 1 ? w[i][k] * d[i][k] : d[i][k]) * s[i];
+        }
+    }
 }
 }  // namespace
 
@@ -116,269 +125,250 @@ __device__ __forceinline__ void n_field(float c, float below, float cy, float cx
 // same padding), 2: PICCS, (1 - ratio) g(f) + ratio g(f - prior) with the z
 // term dropped at the edges like x and y (PICCS.cu:109-157,322-347).  At the
 // low x / y edge the difference is 0; beyond the high edge n is 0
-// (GD_TV.cu:104-114).  kStep false: pass 1 (partials); true: pass 2.
+// (GD_TV.cu:104-114).
 //
-// A workgroup is a 128 x 8 column tile, one wavefront per row, marching along
-// z through a chunk of planes; every lane owns two adjacent columns.  Its f
-// and n values of the previous plane stay in registers (the z neighbours), as
-// do the x neighbours between its two columns; the f plane goes through LDS
-// for the other x - 1 / y - 1 neighbours and the n_x / n_y planes for the
-// x + 1 / y + 1 ones, in 8-byte pairs where both columns need one.  f and n
-// planes are double-buffered so one barrier per plane orders everything:
-// plane p's f is written before it, read after it; its n is written after it
-// and read after the next plane's barrier.  The first lanes also own the halo
-// entries of the f plane (prefetched in the same register ring as the own
-// columns); the last three wavefronts compute the n-plane halo row y0 + 8 and
-// column x0 + 128, one entry per lane (its f of the previous plane kept in a
-// register).
-template <int kKind, bool kStep>
-__global__ __launch_bounds__(kTvThreads) void tv_tile_kernel(const float* __restrict__ f, float* __restrict__ out,
-                                                             TvParams tp, int nx, int ny, int nz,
-                                                             double* __restrict__ partial,
-                                                             const float* __restrict__ scale_in) {
-    constexpr int NF = kKind == 2 ? 2 : 1;
-    constexpr bool kPadZ = kKind != 2;
-    // 16-byte aligned: every lane reads and writes 8-byte pairs (even indices)
-    __shared__ __align__(16) float F[2][NF][kFH * kFW];      // f planes (ring of two), halo of one voxel
-    __shared__ __align__(16) float Nn[2][2][kNH * kNW];  // (combined) n_y (0) and n_x (1) planes (ring of two)
-    const int tid = threadIdx.x, tx = tid & 63, ty = tid >> 6;
-    // tiles in x-fastest order, consecutive ones on one XCD: the halos a tile
-    // reads from its neighbours are then mostly in that XCD's L2
-    const int ntx = (nx + kTX - 1) / kTX, nty = (ny + kTY - 1) / kTY;
-    const int L = xcd_logical_block((int)blockIdx.x, (int)gridDim.x);
-    const int x0 = (L % ntx) * kTX, y0 = ((L / ntx) % nty) * kTY, z0 = (L / (ntx * nty)) * kZC;
-    const int z1 = min(z0 + kZC, nz);
+// A wavefront works alone, without LDS or barriers: a tile of 64 columns (one a lane) and kCore + 4 rows (in
+// registers) marches along z through a chunk of planes.  In step p it reads f of plane p, completes g of plane p - 1
+// and steps it (kUpdate), then completes g' of plane p - 2 from the stepped planes (kNorm); x neighbours come by
+// wavefront shifts.  Both stages need one voxel more on either side, so 60 of the columns and kCore rows are stored.
+// The volume's own edges need no halo: there, loads give copies of the edge voxels, and after the step the copies are
+// made again, under branches that are uniform in the tile.  Loads run two planes ahead through buffer descriptors
+// (planes outside the volume read 0).
+//
+// What bounds it: vector issue, 20 evaluations of n (a square root and a reciprocal each) for 8 stored rows a plane
+// with 3 wavefronts a SIMD; the halo costs 1.5 to 1.9 times the voxels.  20 iterations, two passes and a one-workgroup
+// sum an iteration before and this: 40 x 36 x 42 486 -> 151 us, 128^3 512 -> 363, 190 x 205 x 181 768 -> 528,
+// 256^3 970 -> 960 (its 256 columns fill 5 tiles of 60 badly); PICCS 134 x 157 x 133, 10 iterations, 480 -> 313.
+template <int kKind, int kCore, bool kUpdate, bool kNorm>
+__global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(const float* __restrict__ f, float* __restrict__ out,
+                                                        TvParams tp, int nx, int ny, int nz, int ntx, int nty,
+                                                        int chunk, int ntiles, float alpha, double norm_eps,
+                                                        const double* __restrict__ partial_in, int npartial,
+                                                        double* __restrict__ partial_out) {
+    constexpr int kR = kCore + 4;               // rows with the halo
+    constexpr int NF = kKind == 2 ? 2 : 1;      // fields: f, and f - prior
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned plane_bytes = (unsigned)nx * (unsigned)ny * 4u;
     const long long plane = (long long)nx * ny;
-    const float scale = kStep ? scale_in[0] : 0.0f;
+    auto rsrc = [&](const float* base, int z) {  // a plane; planes outside the volume read 0 and drop stores
+        const bool in = z >= 0 && z < nz;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (in ? z : 0) * plane), (short)0,
+                                                 in ? (int)plane_bytes : 0, 0x00020000);
+    };
+    // alpha / sqrt(sum of the partials + norm_eps), in the same order and so with the same bits in every wavefront
+    float scale = 0.0f;
+    auto read_scale = [&]() {
+        double part[kTvBlocks / 64], sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < kTvBlocks / 64; ++k) part[k] = k * 64 + lane < npartial ? partial_in[k * 64 + lane] : 0.0;
+#pragma unroll
+        for (int k = 0; k < kTvBlocks / 64; ++k) sum += part[k];
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        scale = (float)((double)alpha / sqrt(sum + norm_eps));
+    };
+    double total = 0.0;
+    const int first = xcd_logical_block((int)blockIdx.x, (int)gridDim.x) * kTvWaves + wave;
+    for (int tile = first; tile < ntiles; tile += (int)gridDim.x * kTvWaves) {
+        const int tx = tile % ntx, ty = tile / ntx % nty, tz = tile / (ntx * nty);
+        const int z0 = tz * chunk, z1 = min(z0 + chunk, nz);
+        // columns x0 - 1 .. x0 + 62, of which 60 are stored, but for the volume's edges; rows y0 .. y0 + kR - 1
+        const int x = tx * kTvColumns + lane - 1, y0 = ty * kCore - 2;
+        const bool low_x = tx == 0, high_x = (tx + 1) * kTvColumns + 3 >= nx, low_y = ty == 0, high_y = y0 + kR > ny;
+        const bool core = x >= 0 && x < nx && (lane >= 2 || low_x) && (lane < 62 || high_x);
+        const unsigned xofs = (unsigned)min(max(x, 0), nx - 1) * 4u;
+        unsigned rowofs[kR];
+#pragma unroll
+        for (int r = 0; r < kR; ++r) rowofs[r] = (unsigned)min(max(y0 + r, 0), ny - 1) * (unsigned)nx * 4u;
 
-    // own columns x0 + 2 tx + c, c = 0, 1
-    const int gy = y0 + ty;
-    int own_ofs[2];
-    bool col[2];
+        // per row: f and prior one plane back, prior two back, the z-free part of g of the plane before; the same of
+        // the updated image one plane further back
+        float fp[kR], pp[kR], ppp[kR], sp[kR], up[kR], tpv[kR];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int gx = x0 + 2 * tx + c;
-        col[c] = gx < nx && gy < ny;
-        own_ofs[c] = col[c] ? gy * nx + gx : -1;
-    }
-    const int own_f = f_index(2 * tx, ty), own_n = n_index(2 * tx, ty);  // even: 8-byte aligned pairs
-    // halo entry of the f plane (lanes tid < kFHalo); the other lanes store
-    // their unused halo value to their own first column just before the own
-    // pair, so the store needs no branch (a store under a branch would pull
-    // its load into the branch).  Positions outside the volume read the
-    // nearest voxel: at x = -1 / y = -1 that makes the edge difference exactly
-    // 0 (GD_TV.cu:104-114); beyond the high edges the value only enters n of
-    // columns outside the volume, which is 0.
-    int hf_idx = own_f, hf_ofs = 0;
-    if (tid < kFHalo) {
-        int lx, ly;
-        f_halo_pos(tid, lx, ly);
-        hf_idx = f_index(lx, ly);
-        const int hx = min(max(x0 + lx, 0), nx - 1), hy = min(max(y0 + ly, 0), ny - 1);
-        hf_ofs = hy * nx + hx;
-    }
-    // halo of the n plane, one entry per lane: row kTY, column 2 tx (last
-    // wavefront) and 2 tx + 1 (the one before), and column kTX, row tx (first
-    // kTY lanes of the third-to-last), so no wavefront does more than one extra
-    // n evaluation per plane
-    int hn_lx = -1, hn_ly = -1;
-    if (ty == kTY - 1) {
-        hn_lx = 2 * tx;
-        hn_ly = kTY;
-    } else if (ty == kTY - 2) {
-        hn_lx = 2 * tx + 1;
-        hn_ly = kTY;
-    } else if (ty == kTY - 3 && tx < kTY) {
-        hn_lx = kTX;
-        hn_ly = tx;
-    }
-    const bool hn_on = hn_lx >= 0;
-    int hn_ofs = -1, hn_f = 0, hn_n = 0;
-    bool hn_col = false;
-    if (hn_on) {
-        const int hx = x0 + hn_lx, hy = y0 + hn_ly;
-        hn_col = hx < nx && hy < ny;
-        hn_ofs = hn_col ? hy * nx + hx : -1;
-        hn_f = f_index(hn_lx, hn_ly);
-        hn_n = n_index(hn_lx, hn_ly);
-    }
-
-    auto load = [&](int k, long long idx) -> float {
-        return k == 0 ? f[idx] : f[idx] - tp.prior[idx];
-    };
-    // The image (and prior) of plane p at the lane's two columns and its
-    // f-halo entry, fetched kAhead planes before use into a ring of registers.
-    // The loads are unconditional, from clamped in-bounds addresses, and raw:
-    // the plane mask and the PICCS difference are applied when the slot is
-    // used, so nothing has to wait for a load before then.  Loads and stores
-    // go through a buffer descriptor per plane (a uniform base) with a 32-bit
-    // byte offset per lane (the plane is below 2^30 voxels), so no 64-bit
-    // address arithmetic runs per access.
-    const float* src[2] = {f, tp.prior};
-    const unsigned ob0 = (unsigned)max(own_ofs[0], 0) * 4u, ob1 = (unsigned)max(own_ofs[1], 0) * 4u,
-                   obh = (unsigned)hf_ofs * 4u;
-    const int plane_bytes = (int)(plane * 4);
-    auto rsrc = [&](const float* pl, int bytes) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(pl), (short)0, bytes, 0x00020000);
-    };
-    auto at = [](__amdgpu_buffer_rsrc_t r, unsigned ob) {
-        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, ob, 0, 0));
-    };
-    float ring[kAhead][2][3];  // [slot][image, prior][column 0, column 1, halo]
-    // The zero slice p = nz (the loop never fetches further) is read through
-    // a descriptor of no records: every load of it returns 0, so no select
-    // runs on the loaded values.
-    auto fetch = [&](int p, float (*v)[3]) {
-        const long long base = (long long)min(max(p, 0), nz - 1) * plane;
-        const int bytes = plane_bytes;
+        for (int r = 0; r < kR; ++r) fp[r] = pp[r] = ppp[r] = sp[r] = up[r] = tpv[r] = 0.0f;
+        float ring[2][NF][kR];
+        auto fetch = [&](int z, float (&v)[NF][kR]) {
 #pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            const __amdgpu_buffer_rsrc_t r = rsrc(src[k] + base, bytes);
-            v[k][0] = at(r, ob0);
-            v[k][1] = at(r, ob1);
-            v[k][2] = at(r, obh);
-        }
-    };
-    // field k of entry e of a fetched slot: f, or f - prior for PICCS
-    // (columns outside the volume keep the clamped value: their n is 0)
-    auto field = [&](float (*v)[3], int k, int e, bool pin) -> float {
-        return pin ? (k == 0 ? v[0][e] : v[0][e] - v[1][e]) : 0.0f;
-    };
-    // 8-byte pair stores need col[1] and an 8-aligned address: the lane's
-    // offset parity is fixed, the plane base's is uniform
-    const bool pair_at0 = col[1] && (ob0 & 4u) == 0, pair_at4 = col[1] && (ob0 & 4u) != 0;
-
-    // f of the previous plane: own columns, n-halo entries
-    float fprev[NF][2], hprev[NF];
-    {
-        const int p = z0 - 1;
-        const bool pin = p >= 0;
-        const long long base = (long long)p * plane;
+            for (int k = 0; k < NF; ++k) {
+                const __amdgpu_buffer_rsrc_t b = rsrc(k == 0 ? f : tp.prior, z);
 #pragma unroll
-        for (int k = 0; k < NF; ++k) {
-#pragma unroll
-            for (int c = 0; c < 2; ++c) fprev[k][c] = (pin && own_ofs[c] >= 0) ? load(k, base + own_ofs[c]) : 0.0f;
-            hprev[k] = (pin && hn_on && hn_ofs >= 0) ? load(k, base + hn_ofs) : 0.0f;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) fetch(min(z0 + j, z1), ring[j]);
-    float nprev[2][3];  // (combined) n of the previous plane at the own columns (z, y, x)
-    // sum of g^2 over the lane's (at most 2 x 16) voxels in FP32, then FP64
-    // across lanes and workgroups
-    float acc = 0.0f;
-    // fully unrolled (planes z0 .. z0 + kZC, at most): ring slot jj % kAhead is
-    // a fixed register set and the compiler sees every load it must wait for
-#pragma unroll
-    for (int jj = 0; jj <= kZC; ++jj) {
-        const int j = jj % kAhead;
-        const int p = z0 + jj;
-        if (p > z1) break;
-        const int b = p & 1;
-        const float fpp[2] = {fprev[0][0], fprev[0][1]};  // f at plane p - 1 (the image, also for PICCS)
-        const bool pin = p < nz;
-        float fc[NF][2];
-#pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            fc[k][0] = field(ring[j], k, 0, pin);
-            fc[k][1] = field(ring[j], k, 1, pin);
-            F[b][k][hf_idx] = field(ring[j], k, 2, pin);
-            *reinterpret_cast<float2*>(&F[b][k][own_f]) = make_float2(fc[k][0], fc[k][1]);
-        }
-        // unconditional (a branch around the loads would make the compiler
-        // wait for all of them); past the chunk it re-reads plane z1 from cache
-        fetch(min(p + kAhead, z1), ring[j]);
-        __syncthreads();
-        // n exists in every plane up to the zero slice nz (TV, AwTV) or in the
-        // volume's planes (PICCS); the loop never runs past plane nz
-        const bool pex = kPadZ || p < nz;
-        const bool has_below = p >= 1;
-        const bool ok0 = pex && col[0], ok1 = pex && col[1];
-        // n of the own columns and of the halo entries, combined over the
-        // fields (PICCS: (1 - ratio) n(f) + ratio n(f - prior); g is linear in
-        // n, so one n field goes through LDS; the weight is 1 for one field)
-        float ncur[2][3], hn3[3];
-#pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            const float wk = NF == 1 ? 1.0f : (k == 0 ? 1.0f - tp.ratio : tp.ratio);
-            auto mix = [&](float* acc3, const float* t) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) acc3[q] = k == 0 ? wk * t[q] : fmaf(wk, t[q], acc3[q]);
-            };
-            const float2 up = *reinterpret_cast<const float2*>(&F[b][k][own_f - kFW]);  // y - 1 of both columns
-            const float left = F[b][k][own_f - 1];                                      // x - 1 of column 0
-            float t0[3], t1[3];
-            n_field<kKind>(fc[k][0], fprev[k][0], up.x, left, ok0, has_below, tp, t0[0], t0[1], t0[2]);
-            n_field<kKind>(fc[k][1], fprev[k][1], up.y, fc[k][0], ok1, has_below, tp, t1[0], t1[1], t1[2]);
-            mix(ncur[0], t0);
-            mix(ncur[1], t1);
-            fprev[k][0] = fc[k][0];
-            fprev[k][1] = fc[k][1];
-            if (hn_on) {
-                const float hc = F[b][k][hn_f];
-                float m[3];
-                n_field<kKind>(hc, hprev[k], F[b][k][hn_f - kFW], F[b][k][hn_f - 1], pex && hn_col, has_below, tp,
-                               m[0], m[1], m[2]);
-                mix(hn3, m);
-                hprev[k] = hc;
+                for (int r = 0; r < kR; ++r)
+                    v[k][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, xofs + rowofs[r], 0, 0));
             }
-        }
-        *reinterpret_cast<float2*>(&Nn[b][0][own_n]) = make_float2(ncur[0][1], ncur[1][1]);
-        *reinterpret_cast<float2*>(&Nn[b][1][own_n]) = make_float2(ncur[0][2], ncur[1][2]);
-        if (hn_on) {
-            Nn[b][0][hn_n] = hn3[1];
-            Nn[b][1][hn_n] = hn3[2];
-        }
-        // g at plane p - 1 from the n planes of p - 1 (buffer b ^ 1, complete
-        // since this plane's barrier) and n_z of plane p
-        if (p > z0) {
-            float res[2];
+        };
+        // n of plane z at rows lo .. hi from the plane's values c (and prior c2) and those below; n_z = value * by goes
+        // to done(r, value, by, false), which completes g of the plane before, and the z-free part of g, n_z + n_y +
+        // n_x - n_y(y + 1) - n_x(x + 1), to done(r, value, 1, true) for rows lo .. hi - 1
+        auto differences = [&](int z, auto lo_, auto hi_, const float (&c)[kR], const float (&c2)[kR],
+                               const float (&below)[kR], const float (&below2)[kR], auto&& done) {
+            constexpr int lo = decltype(lo_)::value, hi = decltype(hi_)::value, kB = kTvBatch < hi - lo + 1 ? kTvBatch : hi - lo + 1;
+            const bool has_z = z >= 1 && z < nz;
+            float keep = 0.0f;
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                // n_x at x + 1: the lane's own second column, or the next lane's first
-                const float nxr = c == 0 ? nprev[1][2] : Nn[b ^ 1][1][own_n + 2];
-                const float nyu = Nn[b ^ 1][0][own_n + kNW + c];
-                const float gv = nprev[c][0] + nprev[c][1] + nprev[c][2] - nxr - nyu - ncur[c][0];
-                res[c] = fpp[c] - gv * scale;
-                if (!kStep) acc = fmaf(col[c] ? gv : 0.0f, gv, acc);
-            }
-            if (kStep) {
-                // the pair as one 8-byte store where both columns exist and the
-                // address allows it (col[1] implies col[0])
-                float* o = out + (long long)(p - 1) * plane;
-                const __amdgpu_buffer_rsrc_t r = rsrc(o, plane_bytes);
-                if ((reinterpret_cast<unsigned long long>(o) & 4ull) == 0 ? pair_at0 : pair_at4) {
-                    __builtin_amdgcn_raw_buffer_store_b64(
-                        __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, make_float2(res[0], res[1])),
-                        r, ob0, 0, 0);
+            for (int r0 = lo; r0 <= hi; r0 += kB) {
+                float n[kB][3], s[kB];
+#pragma unroll
+                for (int k = 0; k < NF; ++k) {
+                    float v[kB], b[kB], u[kB], t[kB][3];
+#pragma unroll
+                    for (int i = 0; i < kB; ++i) {
+                        const int r = r0 + i <= hi ? r0 + i : hi;
+                        v[i] = k == 0 ? c[r] : c[r] - c2[r];
+                        b[i] = k == 0 ? below[r] : below[r] - below2[r];
+                        u[i] = k == 0 ? c[r - 1] : c[r - 1] - c2[r - 1];
+                    }
+                    n_field<kKind>(v, b, u, has_z, tp, t, s);
+#pragma unroll
+                    for (int i = 0; i < kB; ++i)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) {
+                            const float m = NF == 2 && q == 0 ? t[i][0] * s[i] : t[i][q];
+                            n[i][q] = NF == 1   ? m
+                                      : k == 0 ? (1.0f - tp.ratio) * m
+                                               : fmaf(tp.ratio, m, n[i][q]);
+                        }
+                }
+                // n_z + n_y.  n is discontinuous where all differences vanish, so another rounding of g than the one results
+                // have always had moves single voxels by 1e-3 of the range after some iterations: here that is the
+                // rounded product, and in every sixteenth plane the fused one.
+                float zy[kB];
+                if (NF == 1 && (z & 15) == 0) {
+#pragma unroll
+                    for (int i = 0; i < kB; ++i) zy[i] = fmaf(n[i][0], s[i], n[i][1]);
                 } else {
-                    if (col[0]) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(res[0]), r, ob0, 0, 0);
-                    if (col[1]) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(res[1]), r, ob1, 0, 0);
+#pragma clang fp contract(off)
+#pragma unroll
+                    for (int i = 0; i < kB; ++i) zy[i] = (NF == 1 ? n[i][0] * s[i] : n[i][0]) + n[i][1];
+                }
+#pragma unroll
+                for (int i = 0; i < kB; ++i) {
+                    const int r = r0 + i;
+                    if (r > hi) break;
+                    if (r > lo) done(r - 1, keep - n[i][1], 1.0f, true);
+                    done(r, n[i][0], NF == 1 ? s[i] : 1.0f, false);
+                    keep = zy[i] + n[i][2] - lane_after(n[i][2]);
+                }
+            }
+        };
+        // the passes' planes: p reads f, p - 1 is updated, p - 2 adds to the norm
+        constexpr int kLead = kUpdate && kNorm ? 1 : 0;
+        const int begin = z0 - kLead, end = z1 + kLead;
+        auto step = [&](int p, float (&v)[NF][kR]) {
+            float u[kR];  // the image whose norm is taken, plane q
+            float cu[kR], cu2[kR];
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                cu[r] = v[0][r];
+                cu2[r] = NF == 2 ? v[NF - 1][r] : 0.0f;
+            }
+            if (kUpdate) {
+                const float alpha_p = p >= 1 && p <= nz ? scale : 0.0f;  // the zero slices stay 0
+                differences(p, Int<1>{}, Int<kR - 1>{}, cu, cu2, fp, pp, [&](int r, float val, float by, bool rest) {
+                    if (rest) {
+                        sp[r] = val;
+                    } else {
+                        u[r] = fmaf(-alpha_p, fmaf(-val, by, sp[r]), fp[r]);
+                    }
+                });
+#pragma unroll
+                for (int r = 1; r < kR - 1; ++r) formed(sp[r]);
+                if (kNorm) {  // copies of the edge voxels beyond the edges, as the loads give them
+                    if (low_y) u[1] = u[2];
+                    if (high_y) {
+#pragma unroll
+                        for (int r = 2; r < kR; ++r)
+                            if (y0 + r >= ny) u[r] = u[r - 1];
+                    }
+                    if (low_x) {
+#pragma unroll
+                        for (int r = 1; r < kR; ++r) {
+                            const float next = lane_after(u[r]);
+                            u[r] = x < 0 ? next : u[r];
+                        }
+                    }
+                    if (high_x) {
+#pragma unroll
+                        for (int r = 1; r < kR; ++r) {
+                            const float before = lane_before(u[r]);
+                            u[r] = x == nx ? before : u[r];
+                        }
+                    }
+                }
+                if (p > z0 && p <= z1) {
+                    const __amdgpu_buffer_rsrc_t b = rsrc(out, p - 1);
+                    if (core) {
+#pragma unroll
+                        for (int r = 2; r < kR - 2; ++r)
+                            if (y0 + r < ny)
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(u[r]), b, xofs + rowofs[r], 0, 0);
+                    }
+                }
+            }
+            if (kNorm) {
+                const int q = kUpdate ? p - 1 : p;
+                const bool counts = q > z0 && q <= z1;
+                if (!kUpdate) {
+#pragma unroll
+                    for (int r = 0; r < kR; ++r) u[r] = cu[r];
+                }
+                float c2[kR];
+#pragma unroll
+                for (int r = 0; r < kR; ++r) c2[r] = kUpdate ? pp[r] : cu2[r];
+                float g[kR];
+                differences(q, Int<2>{}, Int<kR - 2>{}, u, c2, up, ppp, [&](int r, float val, float by, bool rest) {
+                    if (rest) {
+                        tpv[r] = val;
+                    } else if (r < kR - 2) {
+                        g[r] = fmaf(-val, by, tpv[r]);
+                    }
+                });
+                if (high_y) {
+#pragma unroll
+                    for (int r = 3; r < kR - 2; ++r)
+                        if (y0 + r >= ny) g[r] = 0.0f;
+                }
+                float sum = g[2] * g[2];
+#pragma unroll
+                for (int r = 3; r < kR - 2; ++r) sum = fmaf(g[r], g[r], sum);
+                if (counts) total += core ? (double)sum : 0.0;
+#pragma unroll
+                for (int r = 0; r < kR; ++r) {
+                    up[r] = u[r];
+                    ppp[r] = c2[r];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                fp[r] = cu[r];
+                pp[r] = cu2[r];
+            }
+            fetch(min(p + 2, end), v);
+        };
+        {
+            float v[NF][kR];
+            fetch(begin - 1, v);
+            fetch(begin, ring[0]);
+            fetch(min(begin + 1, end), ring[1]);
+            if (kUpdate && tile == first) read_scale();
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                fp[r] = v[0][r];
+                pp[r] = v[NF - 1][r];
+                if (!kUpdate) {
+                    up[r] = fp[r];
+                    ppp[r] = pp[r];
                 }
             }
         }
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) nprev[c][q] = ncur[c][q];
+        for (int p = begin; p <= end; p += 2) {
+            step(p, ring[0]);
+            if (p + 1 <= end) step(p + 1, ring[1]);
+        }
     }
-    if (!kStep) {
-        const double sum = block_sum((double)acc);
-        if (tid == 0)
-            partial[L] = sum;
+    if (kNorm) {
+        const double sum = block_sum(total);
+        if (threadIdx.x == 0) partial_out[blockIdx.x] = sum;
     }
-}
-
-// scale = alpha / sqrt(sum of partials + norm_eps), summed in a fixed order;
-// norm_eps = 1e-7 for TV and AwTV (GD_TV.cu:561), 0 for PICCS (PICCS.cu:370).
-__global__ __launch_bounds__(kTvThreads) void tv_scale_kernel(const double* __restrict__ partial, int npartial,
-                                                              float alpha, double norm_eps, float* __restrict__ scale) {
-    double s = 0.0;
-    // unrolled so the loads are issued together; the additions keep their order
-#pragma unroll 8
-    for (int i = threadIdx.x; i < npartial; i += kTvThreads) s += partial[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) scale[0] = (float)((double)alpha / sqrt(s + norm_eps));
 }
 
 namespace {
@@ -393,30 +383,45 @@ int run_tv_descent(const float* img, float* dst, float alpha, const TvParams& tp
         if (dst != img) TIGRE_HIP_TRY(hipMemcpyAsync(dst, img, n * sizeof(float), hipMemcpyDeviceToDevice, stream));
         return TIGRE_OK;
     }
-    // one tile per workgroup in a 1-D grid (the kernel orders the tiles per XCD)
-    const long long tiles = ((nx + kTX - 1) / kTX) * ((ny + kTY - 1) / kTY) * ((nz + kZC - 1) / kZC);
-    TIGRE_REQUIRE(tiles < (1LL << 31), "image too large");
-    const int nblocks = (int)tiles;
-    const dim3 grid((unsigned)nblocks);
+    const long long ntx = nx <= 63 ? 1 : (nx - 63 + kTvColumns - 1) / kTvColumns + 1;
+    // 8 rows a tile cost the least halo; 2 rows and chunks from 2 planes give a small volume more wavefronts and
+    // shorter ones (20 iterations: 40 x 36 x 42 151 us, 240 with 8 rows; 64^3 180 and 237; 128^3, 1536 tiles of 8
+    // rows, 383 and 363).  Chunks are as long as one round of the chip's slots allows (3 wavefronts a SIMD, 2 for
+    // PICCS; 256^3: 992 us with 3072 tiles, 1139 with 1536, 1145 with 4096).
+    const bool small = ntx * ((ny + 7) / 8) * ((nz + 3) / 4) < 1024;
+    const int rows = small ? 2 : 8;
+    const long long nty = (ny + rows - 1) / rows, slots = kKind == 2 && !small ? 2048 : 3072;
+    const int chunk = (int)std::min(64LL, std::max(small ? 2LL : 4LL, (nz * ntx * nty + slots - 1) / slots));
+    const long long ntiles = ntx * nty * ((nz + chunk - 1) / chunk);
+    TIGRE_REQUIRE(ntiles < (1LL << 30), "image too large");
+    const int nblocks = (int)std::min((long long)kTvBlocks, (ntiles + kTvWaves - 1) / kTvWaves);
     StreamScratch scratch(stream);
     float* buf[2] = {nullptr, nullptr};
-    double* partial = nullptr;
-    float* scale = nullptr;
+    double* partial[2] = {nullptr, nullptr};
     TIGRE_CHECK(scratch.alloc(&buf[0], n * sizeof(float)));
     TIGRE_CHECK(scratch.alloc(&buf[1], n * sizeof(float)));
-    TIGRE_CHECK(scratch.alloc(&partial, (size_t)nblocks * sizeof(double)));
-    TIGRE_CHECK(scratch.alloc(&scale, 256));
+    TIGRE_CHECK(scratch.alloc(&partial[0], 2 * kTvBlocks * sizeof(double)));
+    partial[1] = partial[0] + kTvBlocks;
     const float* src = img;
     int cur = 0;
     for (int it = 0; it < maxiter; ++it) {
-        float* o = (it == maxiter - 1 && dst != img) ? dst : buf[cur];
+        const bool last = it == maxiter - 1;
+        float* o = (last && dst != img) ? dst : buf[cur];
         KernelTimerScope timer(TIGRE_KERNEL_POCS_TV, stream);
-        hipLaunchKernelGGL((tv_tile_kernel<kKind, false>), grid, dim3(kTvThreads), 0, stream, src, nullptr, tp,
-                           (int)nx, (int)ny, (int)nz, partial, nullptr);
-        hipLaunchKernelGGL(tv_scale_kernel, dim3(1), dim3(kTvThreads), 0, stream, partial, nblocks, alpha, norm_eps,
-                           scale);
-        hipLaunchKernelGGL((tv_tile_kernel<kKind, true>), grid, dim3(kTvThreads), 0, stream, src, o, tp, (int)nx,
-                           (int)ny, (int)nz, nullptr, scale);
+#define TIGRE_TV(C, U, N)                                                                                          \
+    hipLaunchKernelGGL((tv_kernel<kKind, C, U, N>), dim3((unsigned)nblocks), dim3(kTvThreads), 0, stream, src, o, tp, \
+                       (int)nx, (int)ny, (int)nz, (int)ntx, (int)nty, chunk, (int)ntiles, alpha, norm_eps,          \
+                       partial[cur], nblocks, partial[(U) ? cur ^ 1 : cur])
+#define TIGRE_TV_ROWS(U, N)             \
+    do {                                \
+        if (rows == 8) TIGRE_TV(8, U, N); \
+        else TIGRE_TV(2, U, N);         \
+    } while (0)
+        if (it == 0) TIGRE_TV_ROWS(false, true);
+        if (last) TIGRE_TV_ROWS(true, false);
+        else TIGRE_TV_ROWS(true, true);
+#undef TIGRE_TV_ROWS
+#undef TIGRE_TV
         TIGRE_HIP_TRY(hipGetLastError());
         src = o;
         cur ^= 1;
@@ -473,14 +478,6 @@ template <int kT>
 struct RofSteps {
     float tau1[kT], tau2[kT];
 };
-
-// Value of the lane before / after this one (0 in lane 0 / 63).
-__device__ __forceinline__ float lane_before(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float lane_after(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xF, 0xF, true));
-}
 
 struct RofP {
     float x, y, z;
