@@ -114,23 +114,19 @@ void build_forward_records(const HostGeometry& g, bool interp, int views_per_gro
     }
     rec->nbeam = (int)rec->ordered.size();
     for (int i : rest) rec->ordered.push_back(views[i]);
-    // Groups of fewer than four views leave view slots of a workgroup empty:
-    // when no group holds more than two views, every workgroup traces twice the
-    // pixels of each of its views, and when every group holds one view, four times,
-    // provided the launch keeps a workgroup for every CU of the 256-CU MI355X (a
-    // single view of a 256 x 256 detector in 64 workgroups measured 0.116 against
-    // 0.058 ms in 16 x 16 tiles; of a 512 x 512 one, in 256, 0.221 against 0.250 ms).
-    // Siddon's tiles are wide along u: the box of a 32 x 8 tile in four views has fewer rows than that of a
-    // 16 x 16 one, and longer ones, which waste less of their 128-byte lines (512^3, 360 views 25.3 against
-    // 26.4 ms; a ragged 200^3 volume with 4-degree spacing, whose 16 x 16 boxes do not fit eight planes, 0.68
-    // against 0.74 ms; one view a group, 64 x 16 against 32 x 32: 512^3, 20 views 3.13 against 3.34 ms).
+    // The tile of a workgroup's views.  Siddon's tiles are wide along u: the box of a 32 x 8 tile in four views has
+    // fewer rows than that of a 16 x 16 one, and longer ones, which waste less of their 128-byte lines (512^3, 360
+    // views 25.3 against 26.4 ms; a ragged 200^3 volume with 4-degree spacing, whose 16 x 16 boxes do not fit eight
+    // planes, 0.68 against 0.74 ms).  Groups of fewer than four views leave view slots empty, and the tile grows to
+    // 32 x 16 where that keeps a workgroup for every CU (a single view of a 256 x 256 detector in 64 workgroups
+    // measured 0.116 against 0.058 ms in 16 x 16 tiles).  It grows no further: with one view a group half of the
+    // wavefronts then only load, but the box is half that of a 64 x 16 or 32 x 32 tile and takes more planes
+    // (Siddon, 227 x 227 x 154, 20 views 0.32 against 0.48 and 0.40 ms, 320^3, 24 views 1.05 against 1.28 and 1.19;
+    // interpolated, 256^3, 20 views 1.04 against 1.21 in 32 x 32, 384^3, 24 views 3.71 against 4.09).
     int most = 0;
     for (int k = 0; k < rec->ngroups(); ++k) most = std::max(most, rec->groups[4 * k + 1]);
     rec->shape = interp ? BeamShape{1, 4} : BeamShape{2, 2};
-    if (most == 1 || most == 2) {
-        const BeamShape more = most == 2 ? BeamShape{2, 4} : (interp ? BeamShape{2, 8} : BeamShape{4, 4});
-        if (beam_job_blocks(g, rec->ngroups(), more) >= 256) rec->shape = more;
-    }
+    if (most <= 2 && beam_job_blocks(g, rec->ngroups(), BeamShape{2, 4}) >= 256) rec->shape = BeamShape{2, 4};
 }
 
 namespace {
