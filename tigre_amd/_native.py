@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 import numpy as np
 
@@ -273,6 +274,13 @@ def check(status: int, where: str) -> None:
     raise TigreCudaCallError(where, status, msg)
 
 
+# The struct's members in C's own order, sizes and alignment, so that one call fills it.
+_PACK = struct.Struct("@" + "".join({ctypes.c_int: "i", ctypes.c_float: "f", _fp: "P"}[t]
+                                    for _, t in TigreGeometry._fields_))
+_PER_VIEW = ("offOrigX", "offOrigY", "offOrigZ", "DSO", "offDetecU", "offDetecV", "DSD", "dRoll", "dPitch", "dYaw",
+             "COR")
+
+
 class CGeometry:
     """A filled ``TigreGeometry`` plus the float32 arrays it points into.
 
@@ -283,36 +291,31 @@ class CGeometry:
     rotDetector[i] = (yaw, pitch, roll)."""
 
     def __init__(self, geo, nangles: int):
-        f32 = lambda a: np.ascontiguousarray(np.asarray(a, dtype=np.float32).reshape(-1))  # noqa: E731
         off = np.asarray(geo.offOrigin, dtype=np.float32).reshape(nangles, 3)
         offd = np.asarray(geo.offDetector, dtype=np.float32).reshape(nangles, 2)
         rot = np.asarray(geo.rotDetector, dtype=np.float32).reshape(nangles, 3)
-        self._keep = {
-            "offOrigX": f32(off[:, 2]), "offOrigY": f32(off[:, 1]), "offOrigZ": f32(off[:, 0]),
-            "DSO": f32(np.broadcast_to(np.asarray(geo.DSO, dtype=np.float32), (nangles,))),
-            "DSD": f32(np.broadcast_to(np.asarray(geo.DSD, dtype=np.float32), (nangles,))),
-            "offDetecU": f32(offd[:, 1]), "offDetecV": f32(offd[:, 0]),
-            "dRoll": f32(rot[:, 2]), "dPitch": f32(rot[:, 1]), "dYaw": f32(rot[:, 0]),
-            "COR": f32(np.broadcast_to(np.asarray(geo.COR, dtype=np.float32), (nangles,))),
-        }
-        s = TigreGeometry()
+        # the per-view fields, one row each
+        rows = np.empty((len(_PER_VIEW), nangles), dtype=np.float32)
+        rows[0:3] = off.T[::-1]
+        for k, name in ((3, "DSO"), (6, "DSD"), (10, "COR")):
+            a = np.asarray(getattr(geo, name), dtype=np.float32)
+            rows[k] = a if a.ndim < 2 else np.broadcast_to(a, (nangles,))
+        rows[4:6] = offd.T[::-1]
+        rows[7:10] = rot.T[::-1]
         nv = [int(x) for x in np.asarray(geo.nVoxel).reshape(3)]
-        sv = np.asarray(geo.sVoxel, dtype=np.float32).reshape(3)
-        dv = np.asarray(geo.dVoxel, dtype=np.float32).reshape(3)
         nd = [int(x) for x in np.asarray(geo.nDetector).reshape(2)]
-        sd = np.asarray(geo.sDetector, dtype=np.float32).reshape(2)
-        dd = np.asarray(geo.dDetector, dtype=np.float32).reshape(2)
-        s.nVoxelX, s.nVoxelY, s.nVoxelZ = nv[2], nv[1], nv[0]
-        s.sVoxelX, s.sVoxelY, s.sVoxelZ = float(sv[2]), float(sv[1]), float(sv[0])
-        s.dVoxelX, s.dVoxelY, s.dVoxelZ = float(dv[2]), float(dv[1]), float(dv[0])
-        s.nDetecU, s.nDetecV = nd[1], nd[0]
-        s.sDetecU, s.sDetecV = float(sd[1]), float(sd[0])
-        s.dDetecU, s.dDetecV = float(dd[1]), float(dd[0])
-        s.unitX = s.unitY = s.unitZ = 1.0
-        s.accuracy = float(np.float32(geo.accuracy))
-        for name, arr in self._keep.items():
-            setattr(s, name, arr.ctypes.data_as(_fp))
-        self.struct = s
+        sv, dv = (np.asarray(a, dtype=np.float32).reshape(3).tolist() for a in (geo.sVoxel, geo.dVoxel))
+        sd, dd = (np.asarray(a, dtype=np.float32).reshape(2).tolist() for a in (geo.sDetector, geo.dDetector))
+        at = rows.ctypes.data
+        step = 4 * nangles
+        v = {name: at + k * step for k, name in enumerate(_PER_VIEW)}
+        v.update(nVoxelX=nv[2], nVoxelY=nv[1], nVoxelZ=nv[0], sVoxelX=sv[2], sVoxelY=sv[1], sVoxelZ=sv[0],
+                 dVoxelX=dv[2], dVoxelY=dv[1], dVoxelZ=dv[0], nDetecU=nd[1], nDetecV=nd[0], sDetecU=sd[1], sDetecV=sd[0],
+                 dDetecU=dd[1], dDetecV=dd[0], unitX=1.0, unitY=1.0, unitZ=1.0,
+                 accuracy=float(np.float32(geo.accuracy)))
+        packed = _PACK.pack(*[v.get(name, 0) for name, _ in TigreGeometry._fields_])
+        self._keep = rows
+        self.struct = TigreGeometry.from_buffer_copy(packed.ljust(ctypes.sizeof(TigreGeometry), b"\0"))
 
     def ptr(self):
         return ctypes.byref(self.struct)

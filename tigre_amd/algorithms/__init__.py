@@ -23,7 +23,7 @@ import time
 import numpy as np
 
 from .. import _native
-from ..geometry import prepared
+from ..geometry import duplicate, prepared
 from ..operators import _stream_handle
 from ..utilities.filtering import filtering, weighted_filtering
 from ..utilities.order_subsets import order_subsets
@@ -45,7 +45,7 @@ def _torch():
 
 def _sub_geometry(geo, idx):
     """Geometry restricted to views idx (iterative_recon_alg.py:335-341)."""
-    g = copy.deepcopy(geo)
+    g = duplicate(geo)
     for a in ("DSD", "DSO", "COR"):
         setattr(g, a, np.asarray(getattr(geo, a))[idx])
     for a in ("offOrigin", "offDetector", "rotDetector"):
@@ -57,37 +57,40 @@ class ViewSets:
     """Projector calls on fixed subsets of views of one geometry.
 
     The per-subset geometry (checked, rounded to float32, converted to the C
-    struct) is prepared once; ``ax``/``atb`` then call the device entry points
-    directly on the current stream."""
+    struct) is prepared once, when the subset is first used; ``ax``/``atb``
+    then call the device entry points directly on the current stream."""
 
     def __init__(self, geo, angles, blocks):
-        self.geo = copy.deepcopy(geo)
+        self.geo = duplicate(geo)
         self.geo.check_geo(angles)
         self.angles = self.geo.angles
         # the reference's Ax / Atb pick the parallel-beam operators from
         # geo.mode (_Ax.pyx:67-87, _Atb.pyx:56-76)
         self.parallel = getattr(self.geo, "mode", "cone") == "parallel"
-        self.sets = []
-        for idx in blocks:
-            idx = np.asarray(idx, dtype=np.int64).reshape(-1)
-            g = prepared(_sub_geometry(self.geo, idx), self.angles[idx])
-            cg = _native.CGeometry(g, len(idx))
-            ang = np.ascontiguousarray(g.angles, dtype=np.float32)
-            self.sets.append((idx, g, cg, ang))
+        self.blocks = [np.asarray(idx, dtype=np.int64).reshape(-1) for idx in blocks]
+        self._sets = [None] * len(self.blocks)
         self.lib = _native.lib()
         self.vol_shape = tuple(int(v) for v in np.asarray(self.geo.nVoxel))
         self.det_shape = (int(self.geo.nDetector[0]), int(self.geo.nDetector[1]))
 
     def __len__(self):
-        return len(self.sets)
+        return len(self.blocks)
 
     def index(self, j):
-        return self.sets[j][0]
+        return self.blocks[j]
+
+    def set(self, j):
+        """(views, geometry, C geometry, float32 angles) of subset j."""
+        if self._sets[j] is None:
+            idx = self.blocks[j]
+            g = prepared(_sub_geometry(self.geo, idx), self.angles[idx])
+            self._sets[j] = (idx, g, _native.CGeometry(g, len(idx)), np.ascontiguousarray(g.angles, dtype=np.float32))
+        return self._sets[j]
 
     def ax(self, img, j, kind=_native.PROJ_SIDDON, out=None):
         """Projections of subset j, stored like ``img`` (float32, bfloat16 or float16)."""
         torch = _torch()
-        idx, g, cg, ang = self.sets[j]
+        idx, g, cg, ang = self.set(j)
         if out is None:
             out = torch.empty((len(idx),) + self.det_shape, dtype=img.dtype, device=img.device)
         fn = self.lib.tigre_ax_parallel_device if self.parallel else self.lib.tigre_ax_device_typed
@@ -100,7 +103,7 @@ class ViewSets:
     def atb(self, proj, j, kind=_native.BACKPROJ_FDK, out=None):
         """Backprojection of subset j, stored like ``proj``."""
         torch = _torch()
-        idx, g, cg, ang = self.sets[j]
+        idx, g, cg, ang = self.set(j)
         if out is None:
             out = torch.empty(self.vol_shape, dtype=proj.dtype, device=proj.device)
         if self.parallel:
@@ -203,7 +206,7 @@ def fdk(proj, geo, angles, filter=None, verbose=False, return_tensor=False, **kw
         p, geo, theta = _wang_padding(p, geo)
         w = torch.as_tensor((2.0 * wang_weights(geo, theta)).astype(np.float32), device=p.device)
         p = p * w
-    g = copy.deepcopy(geo)
+    g = duplicate(geo)
     g.check_geo(angles)
     g.filter = filter
     nV, nU = int(g.nDetector[0]), int(g.nDetector[1])
@@ -248,7 +251,7 @@ class _SartState:
     def __init__(self, proj, geo, angles, blocksize, order=None, init=None, lmbda=1.0, noneg=True, verbose=False,
                  use_plans=True):
         torch = _torch()
-        self.geo = copy.deepcopy(geo)
+        self.geo = duplicate(geo)
         self.geo.check_geo(angles)
         self.angles = self.geo.angles
         _, index = order_subsets(self.angles, blocksize, order)
@@ -288,7 +291,7 @@ class _SartState:
     def _weights_w(self):
         """W = 1 / Ax(ones(2^3)) on an enlarged volume (iterative_recon_alg.py:214-230)."""
         torch = _torch()
-        g = copy.deepcopy(self.geo)
+        g = duplicate(self.geo)
         g.sVoxel = np.asarray(g.sVoxel, dtype=np.float64).copy()
         g.sVoxel[1:] = g.sVoxel[1:] * 1.1
         g.sVoxel[0] = max(g.sDetector[0], g.sVoxel[0])
@@ -307,7 +310,7 @@ class _SartState:
             nY, nX = self.views.vol_shape[1:]
             return torch.stack([torch.full((nY, nX), float(len(idx)), dtype=torch.float32, device="cuda")
                                 for idx in self.blocks])
-        g = copy.deepcopy(self.geo)
+        g = duplicate(self.geo)
         s = np.asarray(g.sVoxel, dtype=np.float64)
         g.sVoxel = s * np.max(s[1:] / np.linalg.norm(s[1:])) * 0.9
         g.dVoxel = g.sVoxel / np.asarray(g.nVoxel)

@@ -149,7 +149,7 @@ bool backward_is_axial(const HostGeometry& g, const std::vector<BwdView>& v);
 // Device helpers (runtime.cpp)
 // ---------------------------------------------------------------------------
 int select_device(const int* gpuids, int ngpus);
-int upload_async(void** d_ptr, const void* host, size_t bytes, hipStream_t stream);
+int upload_async(void** d_ptr, const void* host, size_t bytes, size_t total, hipStream_t stream);
 
 // Stream-ordered scratch of one call: every block allocated through it is
 // released with hipFreeAsync on the same stream when the guard goes out of
@@ -170,8 +170,9 @@ class StreamScratch {
         *p = static_cast<T*>(q);
         return TIGRE_OK;
     }
-    int upload(void** p, const void* host, size_t bytes) {
-        TIGRE_CHECK(upload_async(p, host, bytes, stream_));
+    // A block of total bytes that starts with a copy of the host's bytes.
+    int upload(void** p, const void* host, size_t bytes, size_t total) {
+        TIGRE_CHECK(upload_async(p, host, bytes, total, stream_));
         blocks_.push_back(*p);
         return TIGRE_OK;
     }

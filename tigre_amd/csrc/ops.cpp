@@ -3,6 +3,7 @@
 // caller's stream with stream-ordered scratch allocations.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "common.hpp"
 
@@ -178,19 +179,24 @@ int ax_device(const void* d_img, const HostGeometry& g, void* d_proj_out, int pr
     TIGRE_REQUIRE(valid_dtype(dtype), "unknown storage type");
     const bool interp = projection_type == TIGRE_PROJ_INTERPOLATED;
     StreamScratch scratch(stream);
-    // narrow storage: the kernels write float projections, rounded at the end
     const long long nproj = (long long)g.nDetec[0] * g.nDetec[1] * g.nangles;
-    float* d_proj = static_cast<float*>(d_proj_out);
-    if (dtype != TIGRE_DTYPE_F32) TIGRE_CHECK(scratch.alloc(&d_proj, (size_t)nproj * sizeof(float)));
     ForwardRecords rec;
     build_forward_records(g, interp, 4, &rec);
-    void* d_views = nullptr;
-    void* d_groups = nullptr;
-    TIGRE_CHECK(scratch.upload(&d_views, rec.ordered.data(), rec.ordered.size() * sizeof(FwdView)));
-    if (rec.ngroups() > 0) TIGRE_CHECK(scratch.upload(&d_groups, rec.groups.data(), rec.groups.size() * sizeof(int)));
-    char* ws = nullptr;
-    const size_t wsb = ax_workspace_bytes(g, rec, interp);
-    if (wsb) TIGRE_CHECK(scratch.alloc(&ws, wsb));
+    // One block for the view records, the groups, the workspace and, with narrow storage, the float projections that
+    // the kernels write before they are rounded: one allocation and one copy a call, not four and two.
+    const size_t views_b = rec.ordered.size() * sizeof(FwdView), groups_b = rec.groups.size() * sizeof(int);
+    const size_t groups_at = align256(views_b), ws_at = groups_at + align256(groups_b);
+    const size_t proj_at = ws_at + ax_workspace_bytes(g, rec, interp);
+    const size_t total = proj_at + (dtype == TIGRE_DTYPE_F32 ? 0 : (size_t)nproj * sizeof(float));
+    std::vector<char> records(groups_at + groups_b);
+    std::memcpy(records.data(), rec.ordered.data(), views_b);
+    if (groups_b) std::memcpy(records.data() + groups_at, rec.groups.data(), groups_b);
+    void* block = nullptr;
+    TIGRE_CHECK(scratch.upload(&block, records.data(), records.size(), total));
+    char* base = static_cast<char*>(block);
+    const void *d_views = base, *d_groups = base + groups_at;
+    char* ws = base + ws_at;
+    float* d_proj = dtype == TIGRE_DTYPE_F32 ? static_cast<float*>(d_proj_out) : reinterpret_cast<float*>(base + proj_at);
     TIGRE_CHECK(ax_launch(d_img, dtype, g, rec, (const FwdView*)d_views, (const int*)d_groups, projection_type, layout,
                           d_proj, ws, 8, stream));
     if (dtype != TIGRE_DTYPE_F32) TIGRE_CHECK(launch_store_converted(d_proj, d_proj_out, nproj, dtype, stream));
@@ -220,15 +226,19 @@ int atb_device(const void* d_proj, const HostGeometry& g, void* d_vol_out, int b
     TIGRE_REQUIRE(valid_dtype(dtype), "unknown storage type");
     StreamScratch scratch(stream);
     const long long nvox = (long long)g.nVoxel[0] * g.nVoxel[1] * g.nVoxel[2];
-    float* d_vol = static_cast<float*>(d_vol_out);
-    if (dtype != TIGRE_DTYPE_F32) TIGRE_CHECK(scratch.alloc(&d_vol, (size_t)nvox * sizeof(float)));
     std::vector<BwdView> views;
     backward_views(g, &views);
     const bool axial = backward_is_axial(g, views);
-    void* d_views = nullptr;
-    TIGRE_CHECK(scratch.upload(&d_views, views.data(), views.size() * sizeof(BwdView)));
-    char* ws = nullptr;
-    TIGRE_CHECK(scratch.alloc(&ws, atb_workspace_bytes(g)));
+    // one block: view records, workspace, and the float volume of narrow storage
+    const size_t views_b = views.size() * sizeof(BwdView), ws_at = align256(views_b);
+    const size_t vol_at = ws_at + atb_workspace_bytes(g);
+    void* block = nullptr;
+    TIGRE_CHECK(scratch.upload(&block, views.data(), views_b,
+                               vol_at + (dtype == TIGRE_DTYPE_F32 ? 0 : (size_t)nvox * sizeof(float))));
+    char* base = static_cast<char*>(block);
+    const void* d_views = base;
+    char* ws = base + ws_at;
+    float* d_vol = dtype == TIGRE_DTYPE_F32 ? static_cast<float*>(d_vol_out) : reinterpret_cast<float*>(base + vol_at);
     TIGRE_CHECK(atb_launch(d_proj, dtype, g, (const BwdView*)d_views, axial, backprojection_type, layout, d_vol, ws,
                            16, AtbUpdate{}, stream));
     if (dtype != TIGRE_DTYPE_F32) TIGRE_CHECK(launch_store_converted(d_vol, d_vol_out, nvox, dtype, stream));

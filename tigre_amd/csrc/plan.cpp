@@ -17,18 +17,15 @@ struct TigrePlan_ {
     int device = 0;
     HostGeometry g;
     ForwardRecords fwd[2];              // [0] Siddon, [1] interpolated
-    void* d_fwd[2] = {nullptr, nullptr};
-    void* d_groups[2] = {nullptr, nullptr};
-    void* d_bwd = nullptr;
+    const void* d_fwd[2] = {nullptr, nullptr};
+    const void* d_groups[2] = {nullptr, nullptr};
+    const void* d_bwd = nullptr;
     bool axial = false;
     int max_planes = 8;
     int zper = 16;
+    void* d_tables = nullptr;  // one allocation, every table at a 256-byte boundary
     ~TigrePlan_() {
-        for (int k = 0; k < 2; ++k) {
-            if (d_fwd[k]) (void)hipFree(d_fwd[k]);
-            if (d_groups[k]) (void)hipFree(d_groups[k]);
-        }
-        if (d_bwd) (void)hipFree(d_bwd);
+        if (d_tables) (void)hipFree(d_tables);
     }
 };
 
@@ -126,17 +123,30 @@ int tigre_plan_create(const TigreGeometry* geo, const float* angles, int nangles
         TIGRE_CHECK(import_geometry(geo, angles, nangles, &p->g));
         p->max_planes = max_slab_planes;
         p->zper = slices_per_thread;
-        for (int k = 0; k < 2; ++k) {
-            build_forward_records(p->g, k == 1, views_per_group, &p->fwd[k]);
-            TIGRE_CHECK(upload_sync(&p->d_fwd[k], p->fwd[k].ordered.data(),
-                                    p->fwd[k].ordered.size() * sizeof(FwdView)));
-            TIGRE_CHECK(upload_sync(&p->d_groups[k], p->fwd[k].groups.data(),
-                                    p->fwd[k].groups.size() * sizeof(int)));
-        }
+        for (int k = 0; k < 2; ++k) build_forward_records(p->g, k == 1, views_per_group, &p->fwd[k]);
         std::vector<BwdView> bwd;
         backward_views(p->g, &bwd);
         p->axial = backward_is_axial(p->g, bwd);
-        TIGRE_CHECK(upload_sync(&p->d_bwd, bwd.data(), bwd.size() * sizeof(BwdView)));
+        const void* src[5] = {p->fwd[0].ordered.data(), p->fwd[0].groups.data(), p->fwd[1].ordered.data(),
+                              p->fwd[1].groups.data(), bwd.data()};
+        const size_t sizes[5] = {p->fwd[0].ordered.size() * sizeof(FwdView), p->fwd[0].groups.size() * sizeof(int),
+                                 p->fwd[1].ordered.size() * sizeof(FwdView), p->fwd[1].groups.size() * sizeof(int),
+                                 bwd.size() * sizeof(BwdView)};
+        size_t off[5], total = 0;
+        for (int k = 0; k < 5; ++k) {
+            off[k] = total;
+            total += align256(sizes[k]);
+        }
+        std::vector<char> host(total, 0);
+        for (int k = 0; k < 5; ++k)
+            if (sizes[k]) std::memcpy(host.data() + off[k], src[k], sizes[k]);
+        TIGRE_CHECK(upload_sync(&p->d_tables, host.data(), total));
+        const char* base = static_cast<const char*>(p->d_tables);
+        for (int k = 0; k < 2; ++k) {
+            p->d_fwd[k] = base + off[2 * k];
+            p->d_groups[k] = base + off[2 * k + 1];
+        }
+        p->d_bwd = base + off[4];
         return TIGRE_OK;
     }();
     if (st != TIGRE_OK) {

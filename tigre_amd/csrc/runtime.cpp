@@ -135,7 +135,7 @@ int select_device(const int* gpuids, int ngpus) {
     return TIGRE_OK;
 }
 
-int upload_async(void** d_ptr, const void* host, size_t bytes, hipStream_t stream) {
+int upload_async(void** d_ptr, const void* host, size_t bytes, size_t total, hipStream_t stream) {
     DeviceState* st = nullptr;
     TIGRE_CHECK(current_state(&st));
     std::lock_guard<std::mutex> lock(st->mu);
@@ -150,7 +150,7 @@ int upload_async(void** d_ptr, const void* host, size_t bytes, hipStream_t strea
         st->staging_bytes[slot] = cap;
     }
     std::memcpy(st->staging[slot], host, bytes);
-    TIGRE_HIP_TRY(hipMallocAsync(d_ptr, bytes, stream));
+    TIGRE_HIP_TRY(hipMallocAsync(d_ptr, total, stream));
     TIGRE_HIP_TRY(hipMemcpyAsync(*d_ptr, st->staging[slot], bytes, hipMemcpyHostToDevice, stream));
     TIGRE_HIP_TRY(hipEventRecord(st->done[slot], stream));
     return TIGRE_OK;

@@ -58,13 +58,13 @@ class Geometry(object):
         for name, shape in (("nVoxel", (3,)), ("sVoxel", (3,)), ("dVoxel", (3,))):
             if np.asarray(getattr(self, name)).shape != shape:
                 raise AttributeError("geo.%s.shape should be %s" % (name, shape))
-        if not np.sum(np.abs(np.asarray(self.dVoxel) * np.asarray(self.nVoxel) - np.asarray(self.sVoxel))) < 1e-6:
+        if not np.abs(np.asarray(self.dVoxel) * np.asarray(self.nVoxel) - np.asarray(self.sVoxel)).sum() < 1e-6:
             raise AttributeError("nVoxel*dVoxel is not equal to sVoxel. Check fields.")
         for name, shape in (("nDetector", (2,)), ("sDetector", (2,)), ("dDetector", (2,))):
             if np.asarray(getattr(self, name)).shape != shape:
                 raise AttributeError("geo.%s.shape should be %s" % (name, shape))
-        if not np.sum(np.abs(np.asarray(self.dDetector) * np.asarray(self.nDetector)
-                             - np.asarray(self.sDetector))) < 1e-6:
+        if not np.abs(np.asarray(self.dDetector) * np.asarray(self.nDetector)
+                      - np.asarray(self.sDetector)).sum() < 1e-6:
             raise AttributeError("nDetector*dDetector is not equal to sDetector. Check fields.")
 
         n = self.n_proj
@@ -86,13 +86,15 @@ class Geometry(object):
         geometry.py:142-195."""
         val = getattr(self, attr)
         if isinstance(val, (float, int, np.floating, np.integer)):
-            setattr(self, attr, np.tile(val, n))
+            setattr(self, attr, np.full(n, val))
             return
         if not isinstance(val, np.ndarray):
             raise TypeError("Data type not understood for: geo." + attr + " with type = " + str(type(val)))
         if val.ndim == 1:
             if val.shape in ((3,), (2,)) and attr not in _PER_VIEW_SCALARS:
-                setattr(self, attr, np.tile(val, (n, 1)))
+                rows = np.empty((n, len(val)), dtype=val.dtype)
+                rows[:] = val
+                setattr(self, attr, rows)
             elif val.shape == (1,):
                 setattr(self, attr, np.tile(val, n) if attr in _PER_VIEW_SCALARS else np.tile(val, (n, 1)))
             elif val.shape == (n,):
@@ -107,6 +109,10 @@ class Geometry(object):
         """Round every non-integer value to float32 (integers stay integers)."""
         for attr, val in list(self.__dict__.items()):
             if val is None or attr in _NO_CAST:
+                continue
+            if type(val) is np.ndarray and val.ndim and val.dtype.kind in "fiu":
+                if val.dtype.kind == "f":
+                    setattr(self, attr, val.astype(np.float32))
                 continue
             try:
                 arr = np.array(val)
@@ -226,9 +232,31 @@ def cone_geometry(n_voxel, s_voxel, n_detector, d_detector, DSO, DSD, accuracy=0
     return g
 
 
+def duplicate(geo):
+    """copy.deepcopy(geo), without its per-object bookkeeping for the plain values and arrays a geometry holds."""
+    cls = type(geo)
+    own = ("__deepcopy__", "__getstate__", "__setstate__", "__getnewargs_ex__", "__getnewargs__", "__slots__")
+    if not (isinstance(geo, Geometry) and cls.__new__ is object.__new__ and cls.__setattr__ is object.__setattr__
+            and cls.__reduce_ex__ is object.__reduce_ex__ and cls.__reduce__ is object.__reduce__
+            and not any(m in d for d in (geo.__dict__, *(c.__dict__ for c in cls.__mro__[:-1])) for m in own)):
+        return copy.deepcopy(geo)  # a subclass with a protocol of its own
+    g = cls.__new__(cls)
+    memo = {id(geo): g}
+    new = g.__dict__
+    for attr, val in geo.__dict__.items():
+        kind = type(val)
+        if kind is np.ndarray and val.dtype.kind in "fiub":
+            new[attr] = val.copy(order="K")
+        elif val is None or kind in (float, int, bool, str):
+            new[attr] = val
+        else:
+            new[attr] = copy.deepcopy(val, memo)
+    return g
+
+
 def prepared(geo, angles):
     """Deep copy, check_geo and cast_to_single, as Ax.py:42-49 / Atb.py:15-21 do."""
-    g = copy.deepcopy(geo)
+    g = duplicate(geo)
     g.check_geo(angles)
     g.cast_to_single()
     return g

@@ -15,6 +15,7 @@ type, and all arithmetic is float32.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import numpy as np
@@ -83,7 +84,18 @@ def _storage_code(t):
 def _stream_handle():
     import torch
 
+    if torch.cuda.is_initialized():  # the current stream without a Stream object around it
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _on(device):
+    """torch.cuda.device(device), for nothing when it is the current one."""
+    import torch
+
+    if device.index == torch.cuda.current_device():
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
 
 
 def Ax(img, geo, angles, projection_type="Siddon", **kwargs):
@@ -116,7 +128,7 @@ def Ax(img, geo, angles, projection_type="Siddon", **kwargs):
         src = img.contiguous()
         out = torch.empty((n, nv, nu), dtype=img.dtype, device=img.device)
         fn = lib.tigre_ax_parallel_device if parallel else lib.tigre_ax_device_typed
-        with torch.cuda.device(img.device):
+        with _on(img.device):
             st = fn(ctypes.c_void_p(src.data_ptr()), cg.ptr(), ctypes.c_void_p(out.data_ptr()),
                     ang.ctypes.data_as(ctypes.c_void_p), n, kind, _native.LAYOUT_PYTHON, code, _stream_handle())
         _native.check(st, "TIGRE: Call to Ax failed")
@@ -164,7 +176,7 @@ def Atb(projections, geo, angles, backprojection_type="FDK", **kwargs):
 
         src = projections.contiguous()
         out = torch.empty(vshape, dtype=projections.dtype, device=projections.device)
-        with torch.cuda.device(projections.device):
+        with _on(projections.device):
             if parallel:
                 st = lib.tigre_atb_parallel_device(ctypes.c_void_p(src.data_ptr()), cg.ptr(),
                                                    ctypes.c_void_p(out.data_ptr()),

@@ -13,7 +13,7 @@ import ctypes
 import numpy as np
 
 from . import _native
-from .operators import _gpu_ids, _is_device_tensor, _stream_handle
+from .operators import _gpu_ids, _is_device_tensor, _on, _stream_handle
 
 __all__ = ["minTV", "minimizeTV", "AwminTV", "minPICCS", "tvdenoise", "im3ddenoise"]
 
@@ -33,7 +33,7 @@ def minTV(src, alpha=15.0, maxiter=100, gpuids=None):
             raise TypeError("minTV expects a 3D float32 tensor")
         x = src.contiguous()
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = lib.tigre_pocs_tv_device(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()),
                                           float(alpha), _sizes(x.shape), int(maxiter), _stream_handle())
         _native.check(st, "minimizeTV:POCS_TV:")
@@ -65,7 +65,7 @@ def AwminTV(src, alpha=15.0, maxiter=100, delta=-0.005, gpuids=None):
             raise TypeError("AwminTV expects a 3D float32 tensor")
         x = src.contiguous()
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = lib.tigre_aw_pocs_tv_device(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()),
                                              float(alpha), _sizes(x.shape), int(maxiter), float(delta),
                                              _stream_handle())
@@ -91,7 +91,7 @@ def minPICCS(src, prior, alpha=15.0, maxiter=100, ratio=0.95, gpuids=None):
         if x.dtype != torch.float32 or p.dtype != torch.float32 or x.shape != p.shape or x.dim() != 3:
             raise TypeError("minPICCS expects two 3D float32 tensors of one shape")
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = lib.tigre_piccs_tv_device(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(p.data_ptr()),
                                            ctypes.c_void_p(out.data_ptr()), float(alpha), float(ratio),
                                            _sizes(x.shape), int(maxiter), _stream_handle())
@@ -119,7 +119,7 @@ def tvdenoise(src, maxiter=100, lamda=15.0, gpuids=None, spacing=(1.0, 1.0, 1.0)
 
         x = src.contiguous()
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = lib.tigre_tvdenoising_device(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()),
                                               float(lamda), sp, _sizes(x.shape), int(maxiter), _stream_handle())
         _native.check(st, "tvdenoising:")

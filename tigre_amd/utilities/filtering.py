@@ -14,7 +14,7 @@ import ctypes
 import numpy as np
 
 from .. import _native
-from ..operators import _stream_handle
+from ..operators import _on, _stream_handle
 
 LONGEST = 4096  # elements of the row kernel's longest transform
 
@@ -125,7 +125,7 @@ def _filter_rows(proj, weight, filt, length, scale):
     w = None if weight is None else weight.contiguous()
     response = torch.as_tensor(row_response(filt, length, scale), device=x.device)
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _native.lib().tigre_filter_rows_device(
             ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(w.data_ptr() if w is not None else None),
             ctypes.c_void_p(response.data_ptr()), ctypes.c_void_p(out.data_ptr()), x.shape[0] * x.shape[1], x.shape[1],
