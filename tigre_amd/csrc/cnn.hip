@@ -344,8 +344,8 @@ __global__ __launch_bounds__(kZmThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 // 0..31, 27 used), and y[v] = aux[v] + (sum_tap P[v + tap][tap] + bias[0]).
 // The 32 -> 32 kernel would spend 27 MFMAs per 16 outputs on this layer with 15 of its
 // 16 columns idle; here it is 2 per 16 input voxels.  A workgroup owns a
-// 64 x 4 tile of outputs and a chunk of planes, and marches through the
-// input planes z0 - 1 .. z0 + chunk: for each it computes P over the 66 x 6
+// 64 x 8 tile of outputs and a chunk of planes, and marches through the
+// input planes z0 - 1 .. z0 + chunk: for each it computes P over the 66 x 10
 // halo'd tile into LDS; then every lane (one output column) adds the 9-tap
 // in-plane sum of each dz group to the accumulator of the output plane that
 // group feeds (input plane z feeds z + 1 with the dz = -1 taps, z with dz = 0,
@@ -353,18 +353,24 @@ __global__ __launch_bounds__(kZmThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 // Every output sums its groups in the order dz = -1, 0, +1 and each group in
 // (dy, dx) order: the result does not depend on the launch shape.  The next
 // plane's A fragments are loaded while the current plane is summed.
-constexpr int kOutTX = 64, kOutTY = 4, kOutZ = 16;  // kOutZ: planes per workgroup, at most
+//
+// What bounds it: reading the 64 bytes a voxel, 1.29 times with the halo of 8
+// rows.  128^3: 40 us, 56 with tiles of 4 rows (1.55 times) and four-byte LDS
+// writes; 8 x 32^3: 14 us.
+constexpr int kOutTX = 64, kOutTY = 8, kOutZ = 16;  // kOutZ: planes per workgroup, at most
 constexpr int kOutHX = kOutTX + 2, kOutHY = kOutTY + 2;
-constexpr int kOutU = kOutHX * kOutHY;           // halo'd voxels per plane (396)
-constexpr int kOutBlocks = (kOutU + 15) / 16;     // MFMA row blocks per plane (25)
-constexpr int kOutPerWave = (kOutBlocks + 3) / 4; // row blocks per wavefront, at most (7)
-constexpr int kOutStride = kOutBlocks * 16 + 1;   // LDS row stride of one tap (odd: conflict-free writes)
+constexpr int kOutU = kOutHX * kOutHY;           // halo'd voxels per plane (660)
+constexpr int kOutBlocks = (kOutU + 15) / 16;     // MFMA row blocks per plane (42)
+constexpr int kOutPerWave = (kOutBlocks + kOutTY - 1) / kOutTY;  // row blocks per wavefront (one a tile row), at most (6)
+// LDS row stride of one tap: an odd number of 16-byte pieces, so the 16 lanes of a write meet all banks
+constexpr int kOutStride = kOutBlocks * 16 + 4;
+static_assert(kOutStride / 4 % 2 == 1, "conflict-free writes");
 
-__global__ __launch_bounds__(256) void conv_out_kernel(const unsigned short* __restrict__ x,
+__global__ __launch_bounds__(64 * kOutTY) void conv_out_kernel(const unsigned short* __restrict__ x,
                                                        const unsigned short* __restrict__ w,
                                                        const float* __restrict__ bias, const float* __restrict__ aux,
                                                        float* __restrict__ y, int N, int D, int H, int W, int chunk) {
-    __shared__ float P[27 * kOutStride];  // [tap][halo'd voxel]
+    __shared__ __align__(16) float P[27 * kOutStride];  // [tap][halo'd voxel]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m = lane & 15, q = lane >> 4;
     const int x0 = blockIdx.x * kOutTX, y0 = blockIdx.y * kOutTY;
@@ -382,11 +388,11 @@ __global__ __launch_bounds__(256) void conv_out_kernel(const unsigned short* __r
         if (tap < 27) raw = *reinterpret_cast<const uint4*>(w + (long long)tap * kC * kC + 8 * q);
         b[hb] = __builtin_bit_cast(bf16x8, raw);
     }
-    // A fragments of plane z: row block wave + 4 k, voxel 16 (wave + 4 k) + m, channels 8 q ..
+    // A fragments of plane z: row block wave + kOutTY k, voxel 16 (wave + kOutTY k) + m, channels 8 q ..
     auto load_plane = [&](int z, bf16x8* a) {
 #pragma unroll
         for (int k = 0; k < kOutPerWave; ++k) {
-            const int u = 16 * (wave + 4 * k) + m;
+            const int u = 16 * (wave + kOutTY * k) + m;
             const int ux = u % kOutHX, uy = u / kOutHX;
             const int gx = x0 - 1 + ux, gy = y0 - 1 + uy;
             const bool ok = u < kOutU && gx >= 0 && gx < W && gy >= 0 && gy < H && z >= 0 && z < D;
@@ -405,17 +411,14 @@ __global__ __launch_bounds__(256) void conv_out_kernel(const unsigned short* __r
         if (zi >= 0 && zi < D) {  // uniform per workgroup
 #pragma unroll
             for (int k = 0; k < kOutPerWave; ++k) {
-                const int blk = wave + 4 * k;
+                const int blk = wave + kOutTY * k;
                 if (blk >= kOutBlocks) break;  // uniform per wavefront
                 const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
                 const f32x4 r0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k], b[0], zero, 0, 0, 0);
                 const f32x4 r1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k], b[1], zero, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int u = 16 * blk + 4 * q + r;
-                    P[m * kOutStride + u] = r0[r];
-                    if (16 + m < 27) P[(16 + m) * kOutStride + u] = r1[r];
-                }
+                const int u = 16 * blk + 4 * q;
+                *reinterpret_cast<f32x4*>(&P[m * kOutStride + u]) = r0;
+                if (16 + m < 27) *reinterpret_cast<f32x4*>(&P[(16 + m) * kOutStride + u]) = r1;
             }
             __syncthreads();  // P complete
             if (zi + 1 <= z1) load_plane(zi + 1, a);
@@ -453,40 +456,65 @@ __global__ __launch_bounds__(256) void conv_out_kernel(const unsigned short* __r
 
 // Convolution of a single FP32 channel (the image, or the loss gradient) into
 // 32 channels.  With one input channel the GEMM k dimension of conv_kernel
-// holds 1 useful channel of 32; here k is the tap instead: A[v][k] =
-// x[v + tap k] (k < 27, zero above), B[k][o] = w[k][o][0], so one MFMA covers
-// all taps of 16 voxels and 16 output channels.  The workgroup's 3 x 6 x 130
-// block of the input is staged in LDS (zero outside the volume) and every
-// lane gathers its 8 taps of each tile from there.
+// holds 1 useful channel of 32; here k is the tap instead: A[o][k] =
+// w[k][o][0] (k < 27, zero above), B[k][v] = x[v + tap k], so one MFMA covers
+// all taps of 16 voxels and 16 output channels, and with the channels as rows a
+// lane ends with eight consecutive channels of a voxel: one 16-byte store.  A
+// workgroup owns 128 x 4 outputs and marches along z through a chunk of planes:
+// the weights' scattered two-byte loads are paid once a chunk, and three planes
+// of the input (6 x 130, zero outside the volume) stay in an LDS ring, from
+// which every lane gathers its 8 taps of each tile.
+//
+// What bounds it: the 64 bytes a voxel it writes.  128^3: 43 us (58 with a
+// workgroup a plane and two-byte stores; the stores alone 53), 8 x 32^3: 17 us
+// (24; with the mask 19, was 25).
 template <int kEpi>
 __global__ __launch_bounds__(256) void conv_taps_kernel(const float* __restrict__ x,
                                                         const unsigned short* __restrict__ w,
                                                         const float* __restrict__ bias, const void* __restrict__ aux,
-                                                        void* __restrict__ y, int N, int D, int H, int W) {
-    constexpr int kPlane = kLdsRows * kLdsBX;
-    __shared__ unsigned short blk[3 * kPlane];  // [dz][row][voxel], rounded to bf16 once when staged
+                                                        void* __restrict__ y, int N, int D, int H, int W, int chunk, bool wide) {
+    constexpr int kPlane = kLdsRows * kLdsBX, kStage = (kPlane + 255) / 256;
+    // [plane % 3][row][voxel], rounded to bf16 once when staged; then zeros for the taps past the 27
+    __shared__ unsigned short blk[3 * kPlane + 16 * kLdsTiles];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m = lane & 15, q = lane >> 4;
     const int x0 = blockIdx.x * (16 * kLdsTiles), y0 = blockIdx.y * 4;
-    const int zz0 = (int)(blockIdx.z % (unsigned)D);
-    const long long n = blockIdx.z / (unsigned)D;
+    const int nchunk = (D + chunk - 1) / chunk;
+    const int z0 = (int)(blockIdx.z % (unsigned)nchunk) * chunk, z1 = min(z0 + chunk, D);
+    const long long n = blockIdx.z / (unsigned)nchunk;
     const int yo = y0 + wave;
 
-    for (int i = tid; i < 3 * kPlane; i += 256) {
-        const int pz = i / kPlane, r = i - pz * kPlane, yi = r / kLdsBX, xi = r - yi * kLdsBX;
-        const int gz = zz0 - 1 + pz, gy = y0 - 1 + yi, gx = x0 - 1 + xi;
-        float v = 0.0f;
-        if (gz >= 0 && gz < D && gy >= 0 && gy < H && gx >= 0 && gx < W)
-            v = x[((n * D + gz) * H + gy) * (long long)W + gx];
-        blk[i] = bf16_bits(v);
+    // plane z of the block: this lane's entries, into registers and then into its LDS slot
+    unsigned from[kStage];
+#pragma unroll
+    for (int k = 0; k < kStage; ++k) {
+        const int i = tid + 256 * k, yi = i / kLdsBX, xi = i - yi * kLdsBX;
+        const int gy = y0 - 1 + yi, gx = x0 - 1 + xi;
+        from[k] = i < kPlane && gy >= 0 && gy < H && gx >= 0 && gx < W ? (unsigned)gy * (unsigned)W + (unsigned)gx : ~0u;
     }
-    // this lane's output channels m and 16 + m
-    float bias_lane[2] = {0.0f, 0.0f};
-    if (kEpi == TIGRE_CNN_EPI_BIAS_RELU) {
-        bias_lane[0] = bias[m];
-        bias_lane[1] = bias[16 + m];
+    auto load = [&](int z, float (&v)[kStage]) {
+        const float* src = x + (n * D + z) * ((long long)H * W);
+#pragma unroll
+        for (int k = 0; k < kStage; ++k) v[k] = z >= 0 && z < D && from[k] != ~0u ? src[from[k]] : 0.0f;
+    };
+    auto keep = [&](int slot, const float (&v)[kStage]) {
+#pragma unroll
+        for (int k = 0; k < kStage; ++k)
+            if (tid + 256 * k < kPlane) blk[slot * kPlane + tid + 256 * k] = bf16_bits(v[k]);
+    };
+    float next[kStage];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {  // planes z0 - 1 .. z0 + 1 into slots 0 .. 2
+        load(z0 - 1 + p, next);
+        keep(p, next);
     }
-    // B fragments: k = 8 q + j is the tap, column o = 16 hb + m
+    if (tid < 16 * kLdsTiles) blk[3 * kPlane + tid] = 0;
+    // this lane's output channels 8 q .. 8 q + 7
+    float bias_lane[8];
+#pragma unroll
+    for (int o = 0; o < 8; ++o) bias_lane[o] = kEpi == TIGRE_CNN_EPI_BIAS_RELU ? bias[8 * q + o] : 0.0f;
+    // A fragments: k = 8 q + j is the tap, row m of product hb the channel 8 (m / 4) + 4 hb + m % 4, so that the two
+    // products leave a lane with eight consecutive channels of one voxel
     bf16x8 b[2];
 #pragma unroll
     for (int hb = 0; hb < 2; ++hb) {
@@ -494,65 +522,80 @@ __global__ __launch_bounds__(256) void conv_taps_kernel(const float* __restrict_
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int tap = 8 * q + j;
-            bits[j] = tap < 27 ? w[((long long)tap * kC + 16 * hb + m) * kC] : (unsigned short)0;
+            bits[j] = tap < 27 ? w[((long long)tap * kC + 8 * (m >> 2) + 4 * hb + (m & 3)) * kC] : (unsigned short)0;
         }
         const uint4 raw = make_uint4(bits[0] | ((unsigned)bits[1] << 16), bits[2] | ((unsigned)bits[3] << 16),
                                      bits[4] | ((unsigned)bits[5] << 16), bits[6] | ((unsigned)bits[7] << 16));
         b[hb] = __builtin_bit_cast(bf16x8, raw);
     }
-    // this lane's taps: offsets in the block relative to (row wave, voxel m) of tile 0
+    // this lane's taps: offsets in the block relative to (row wave, voxel m) of tile 0, for the first output plane;
+    // a plane further, its input planes are one slot further in the ring
     int toff[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int tap = 8 * q + j;
         const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;  // each + 1
-        toff[j] = tap < 27 ? (dz * kLdsRows + wave + dy) * kLdsBX + m + dx : -1;
+        toff[j] = tap < 27 ? (dz * kLdsRows + wave + dy) * kLdsBX + m + dx : 3 * kPlane + m;
     }
-    __syncthreads();
-
-    if (yo >= H) return;
-    const long long obase = ((n * D + zz0) * H + yo) * (long long)W;
-    // one tile at a time (its MFMA pair, then its stores), so few registers are live and several
-    // workgroups share a CU; a workgroup whose tiles lie inside the volume along x stores without
-    // per-voxel tests
-    auto run = [&](auto full_tag) {
-        constexpr bool kFull = decltype(full_tag)::value;
+    for (int z = z0; z < z1; ++z) {
+        __syncthreads();  // the planes of z are in LDS
+        if (z + 1 < z1) load(z + 2, next);
+        const long long obase = ((n * D + z) * H + yo) * (long long)W;
+        // one tile at a time (its MFMA pair, then its store), so few registers are live and several workgroups share a CU
 #pragma unroll
         for (int t = 0; t < kLdsTiles; ++t) {
+            if (x0 + 16 * t >= W || yo >= H) break;
             unsigned short bits[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bits[j] = toff[j] >= 0 ? blk[toff[j] + 16 * t] : (unsigned short)0;
+            for (int j = 0; j < 8; ++j) bits[j] = blk[toff[j] + 16 * t];
             const uint4 raw = make_uint4(bits[0] | ((unsigned)bits[1] << 16), bits[2] | ((unsigned)bits[3] << 16),
                                          bits[4] | ((unsigned)bits[5] << 16), bits[6] | ((unsigned)bits[7] << 16));
             const bf16x8 a = __builtin_bit_cast(bf16x8, raw);
             f32x4 acc[2];
-            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[1], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0], a, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1], a, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            const int xo = x0 + 16 * t + m;
+            if (xo >= W) continue;
+            const long long at = (obase + xo) * kC + 8 * q;
+            unsigned short mask[8], out[8];
+            if (kEpi == TIGRE_CNN_EPI_RELU_MASK) {
+                const unsigned short* am = static_cast<const unsigned short*>(aux) + at;
+                if (wide) {
+                    const uint4 m4 = *reinterpret_cast<const uint4*>(am);
+                    const unsigned word[4] = {m4.x, m4.y, m4.z, m4.w};
 #pragma unroll
-            for (int hb = 0; hb < 2; ++hb) {
-                const int o = hb * 16 + m;
+                    for (int o = 0; o < 8; ++o) mask[o] = (unsigned short)(word[o >> 1] >> (16 * (o & 1)));
+                } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int xo = x0 + 16 * t + 4 * q + r;
-                    if (!kFull && xo >= W) continue;
-                    const long long vox = obase + xo;
-                    float v = acc[hb][r];
-                    if (kEpi == TIGRE_CNN_EPI_BIAS_RELU) {
-                        v += bias_lane[hb];
-                        v = v > 0.0f ? v : 0.0f;
-                    } else {
-                        const unsigned short am = static_cast<const unsigned short*>(aux)[vox * kC + o];
-                        v = (am != 0 && (am & 0x8000u) == 0) ? v : 0.0f;  // activation > 0
-                    }
-                    static_cast<unsigned short*>(y)[vox * kC + o] = bf16_bits(v);
+                    for (int o = 0; o < 8; ++o) mask[o] = am[o];
                 }
             }
+#pragma unroll
+            for (int o = 0; o < 8; ++o) {
+                float v = acc[o >> 2][o & 3];
+                if (kEpi == TIGRE_CNN_EPI_BIAS_RELU) {
+                    v += bias_lane[o];
+                    v = v > 0.0f ? v : 0.0f;
+                } else {
+                    v = (mask[o] != 0 && (mask[o] & 0x8000u) == 0) ? v : 0.0f;  // activation > 0
+                }
+                out[o] = bf16_bits(v);
+            }
+            unsigned short* ym = static_cast<unsigned short*>(y) + at;
+            if (wide) {
+                *reinterpret_cast<uint4*>(ym) = make_uint4(out[0] | ((unsigned)out[1] << 16), out[2] | ((unsigned)out[3] << 16),
+                                                           out[4] | ((unsigned)out[5] << 16), out[6] | ((unsigned)out[7] << 16));
+            } else {
+#pragma unroll
+                for (int o = 0; o < 8; ++o) ym[o] = out[o];
+            }
         }
-    };
-    if (x0 + 16 * kLdsTiles <= W)
-        run(std::true_type{});
-    else
-        run(std::false_type{});
+        __syncthreads();  // plane z - 1 is no longer read
+        if (z + 1 < z1) keep((z - z0) % 3, next);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (8 * q + j < 27) toff[j] += toff[j] < 2 * kPlane ? kPlane : -2 * kPlane;
+    }
 }
 
 // Weight gradient: dw[tap][o][i] = sum_v x[v + tap][i] dy[v][o], one GEMM per tap with k = voxels.
@@ -847,22 +890,27 @@ int launch_cnn_conv(const void* x, int x_mode, const unsigned short* w, const fl
         } else {
             TIGRE_REQUIRE((H + kOutTY - 1) / kOutTY <= 65535, "volume too large for one launch");
             const unsigned ox = (unsigned)((W + kOutTX - 1) / kOutTX), oy = (unsigned)((H + kOutTY - 1) / kOutTY);
-            const int ochunk = march_chunk(N, D, (long long)ox * oy, kOutZ, 768);
+            const int ochunk = march_chunk(N, D, (long long)ox * oy, kOutZ, 512);
             const dim3 ogrid(ox, oy, (unsigned)(N * ((D + ochunk - 1) / ochunk)));
-            hipLaunchKernelGGL(conv_out_kernel, ogrid, dim3(256), 0, stream, xa, w, bias,
+            hipLaunchKernelGGL(conv_out_kernel, ogrid, dim3(64 * kOutTY), 0, stream, xa, w, bias,
                                static_cast<const float*>(aux), static_cast<float*>(y), N, D, H, W, ochunk);
         }
     } else {
         TIGRE_REQUIRE((long long)N * D <= 65535, "too many planes for one launch");
         const float* xf = static_cast<const float*>(x);
-        const dim3 lgrid((unsigned)((W + 16 * kLdsTiles - 1) / (16 * kLdsTiles)), (unsigned)((H + 3) / 4),
-                         (unsigned)(N * D));
+        const unsigned lx = (unsigned)((W + 16 * kLdsTiles - 1) / (16 * kLdsTiles)), ly = (unsigned)((H + 3) / 4);
+        const int chunk = march_chunk(N, D, (long long)lx * ly, 16, 1024);
+        const dim3 lgrid(lx, ly, (unsigned)(N * ((D + chunk - 1) / chunk)));
+        TIGRE_REQUIRE((long long)H * W < 4294967295LL, "plane too large");  // 32-bit offsets in a plane
+        // 16-byte stores and mask loads where the pointers allow them
+        const uintptr_t mask_at = epi == TIGRE_CNN_EPI_RELU_MASK ? reinterpret_cast<uintptr_t>(aux) : 0;
+        const bool wide = ((reinterpret_cast<uintptr_t>(y) | mask_at) & 15) == 0;
         if (epi == TIGRE_CNN_EPI_BIAS_RELU)
             hipLaunchKernelGGL((conv_taps_kernel<TIGRE_CNN_EPI_BIAS_RELU>), lgrid, dim3(256), 0, stream, xf, w, bias,
-                               aux, y, N, D, H, W);
+                               aux, y, N, D, H, W, chunk, wide);
         else if (epi == TIGRE_CNN_EPI_RELU_MASK)
             hipLaunchKernelGGL((conv_taps_kernel<TIGRE_CNN_EPI_RELU_MASK>), lgrid, dim3(256), 0, stream, xf, w, bias,
-                               aux, y, N, D, H, W);
+                               aux, y, N, D, H, W, chunk, wide);
         else TIGRE_CONV(TIGRE_CNN_IN_F32X1, TIGRE_CNN_EPI_RESIDUAL);
     }
 #undef TIGRE_CONV
