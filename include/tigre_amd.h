@@ -173,6 +173,10 @@ int tigre_atb_parallel_device(const void* d_proj, const TigreGeometry* geo, void
 int tigre_filter_rows_device(const float* d_rows, const float* d_weight, const float* d_response,
                              float* d_out, long long rows, int nV, int nU, int log2_len, void* stream);
 
+/* The cone-beam cosine weight dsd / sqrt(dsd^2 + x^2 + y^2) of an nV x nU
+ * detector centred on the axis, pixels of dV x dU, FP64 rounded to float. */
+int tigre_cosine_weight_device(float* d_weight, int nV, int nU, double dV, double dU, double dsd, void* stream);
+
 /* maxIter TV steepest-descent steps on a device volume (X fastest); d_dst may
  * equal d_img.  image_size = {X, Y, Z}. */
 int tigre_pocs_tv_device(const float* d_img, float* d_dst, float alpha, const long* image_size,

@@ -76,3 +76,22 @@ def test_filter_kernel(cuda, n_u):
     y = w.expand(2, 3, n_u).clone().requires_grad_()
     F.filtering(y, geo, angles).sum().backward()
     assert y.grad is not None and bool(torch.isfinite(y.grad).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,pixel", [((1, 1), (0.8, 0.8)), ((3, 257), (1.3, 0.7)), ((129, 64), (1 / 3, 2.1))])
+def test_cosine_weight(cuda, shape, pixel):
+    """The bits of the FP64 expression, rounded once."""
+    import ctypes
+
+    import torch
+
+    from tigre_amd import _native
+
+    dsd = 1536.1
+    w = torch.empty(shape, device=cuda)
+    _native.check(_native.lib().tigre_cosine_weight_device(ctypes.c_void_p(w.data_ptr()), *shape, *pixel, dsd, None), "w")
+    torch.cuda.synchronize()
+    yy, xx = ((np.arange(n) - n / 2 + 0.5) * d for n, d in zip(shape, pixel))
+    ref = (dsd / np.sqrt(dsd ** 2 + xx[None, :] ** 2 + yy[:, None] ** 2)).astype(np.float32)
+    assert np.array_equal(w.cpu().numpy(), ref)

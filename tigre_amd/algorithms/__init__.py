@@ -24,7 +24,7 @@ import numpy as np
 
 from .. import _native
 from ..geometry import duplicate, prepared
-from ..operators import _stream_handle
+from ..operators import _on, _stream_handle
 from ..utilities.filtering import filtering, weighted_filtering
 from ..utilities.order_subsets import order_subsets
 
@@ -212,10 +212,10 @@ def fdk(proj, geo, angles, filter=None, verbose=False, return_tensor=False, **kw
     nV, nU = int(g.nDetector[0]), int(g.nDetector[1])
     dV, dU = float(g.dDetector[0]), float(g.dDetector[1])
     DSD0 = float(np.asarray(g.DSD).reshape(-1)[0])
-    xv = (np.arange(nU) - nU / 2 + 0.5) * dU
-    yv = (np.arange(nV) - nV / 2 + 0.5) * dV
-    xx, yy = np.meshgrid(xv, yv)
-    w = torch.as_tensor((DSD0 / np.sqrt(DSD0 ** 2 + xx ** 2 + yy ** 2)).astype(np.float32), device=p.device)
+    w = torch.empty((nV, nU), dtype=torch.float32, device=p.device)
+    with _on(p.device):
+        _native.check(_native.lib().tigre_cosine_weight_device(ctypes.c_void_p(w.data_ptr()), nV, nU, dV, dU, DSD0,
+                                                               _stream_handle()), "TIGRE: cosine weight failed")
     filt = weighted_filtering(p, w, g, g.angles)
     vs = ViewSets(g, g.angles, [np.arange(len(g.angles))])
     return _result(vs.atb(filt, 0, _native.BACKPROJ_FDK), return_tensor)

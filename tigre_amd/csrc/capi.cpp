@@ -250,6 +250,12 @@ int tigre_filter_rows_device(const float* d_rows, const float* d_weight, const f
     return launch_filter_rows(d_rows, d_weight, d_response, d_out, rows, nV, nU, log2_len, (hipStream_t)stream);
 }
 
+int tigre_cosine_weight_device(float* d_weight, int nV, int nU, double dV, double dU, double dsd, void* stream) {
+    set_error("");
+    TIGRE_REQUIRE(d_weight != nullptr, "null argument");
+    return launch_cosine_weight(d_weight, nV, nU, dV, dU, dsd, (hipStream_t)stream);
+}
+
 int tigre_pocs_tv_device(const float* d_img, float* d_dst, float alpha, const long* image_size, int maxIter,
                          void* stream) {
     set_error("");

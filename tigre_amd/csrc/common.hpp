@@ -250,6 +250,7 @@ int launch_atb(const float* quads, const HostGeometry& g, const BwdView* d_views
 constexpr int kFilterMinLog = 6, kFilterMaxLog = 12;
 int launch_filter_rows(const float* in, const float* weight, const float* response, float* out, long long rows, int nV,
                        int nU, int log2_len, hipStream_t stream);
+int launch_cosine_weight(float* w, int nV, int nU, double dV, double dU, double dsd, hipStream_t stream);
 int run_pocs_tv(const float* img, float* dst, float alpha, long nx, long ny, long nz, int maxiter,
                 hipStream_t stream);
 int run_aw_pocs_tv(const float* img, float* dst, float alpha, float delta, long nx, long ny, long nz, int maxiter,

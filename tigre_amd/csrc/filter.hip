@@ -234,6 +234,29 @@ __global__ __launch_bounds__(Shape<kLog>::kThreads) void filter_rows_kernel(cons
     }
 }
 
+// Cosine weight of every pixel, dsd / sqrt(dsd^2 + x^2 + y^2), in FP64 and rounded once, with the roundings of that
+// expression evaluated left to right.  In place of an upload: 64 K pixels take 2 us, and the host has nothing to wait
+// for.
+__global__ __launch_bounds__(256) void cosine_weight_kernel(float* __restrict__ w, int nV, int nU, double dV, double dU,
+                                                            double dsd) {
+#pragma clang fp contract(off)
+    const long long total = (long long)nV * nU;
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
+        const int v = (int)(i / nU), u = (int)(i - (long long)v * nU);
+        const double x = (u - nU / 2.0 + 0.5) * dU, y = (v - nV / 2.0 + 0.5) * dV;
+        w[i] = (float)(dsd / sqrt(dsd * dsd + x * x + y * y));
+    }
+}
+
+int launch_cosine_weight(float* w, int nV, int nU, double dV, double dU, double dsd, hipStream_t stream) {
+    TIGRE_REQUIRE(nV > 0 && nU > 0, "cosine weight: detector sizes must be positive");
+    const long long blocks = ((long long)nV * nU + 255) / 256;
+    hipLaunchKernelGGL(cosine_weight_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream, w, nV,
+                       nU, dV, dU, dsd);
+    TIGRE_HIP_TRY(hipGetLastError());
+    return TIGRE_OK;
+}
+
 int launch_filter_rows(const float* in, const float* weight, const float* response, float* out, long long rows, int nV,
                        int nU, int log2_len, hipStream_t stream) {
     TIGRE_REQUIRE(rows > 0 && nV > 0 && nU > 0, "filter: rows and detector sizes must be positive");
