@@ -217,8 +217,7 @@ int launch_ax_siddon(const float* bricked, const HostGeometry& g, const BrickGri
 // Beam-staged Siddon (ax_beam.hip).  Staging copy for principal axis P
 // (0 = x, 1 = y): [p][z][a] with a zero border, a = the other horizontal axis.
 long long stage_elements(const HostGeometry& g, int principal);
-int launch_stage_volume(const void* vol, int dtype, const HostGeometry& g, int principal, float* stage,
-                        hipStream_t stream);
+int launch_stage_volume(const void* vol, int dtype, const HostGeometry& g, float* const* stage, hipStream_t stream);
 // The rays of a beam workgroup: a tile of units_u x units_v units of 16 x 4 pixels in each of
 // 16 / (units_u units_v) views.
 struct BeamShape {
@@ -294,10 +293,11 @@ int launch_sart_residual(const float* proj, const float* w, float* ax, long long
 // problems.  Job j owns the blocks [begin, begin + its block count) of the
 // 1-D grid; jobs are sorted by begin, the first begins at 0.
 // ---------------------------------------------------------------------------
-struct StageJob {    // staging copy of an FP32 volume for principal axis `principal`
+struct StageJob {    // staging copies of an FP32 volume for principal axes x and y (null: not used)
     const float* vol;
-    float* out;
-    int nx, ny, nz, principal, na_pad, gx, gy, begin;  // grid (gx, gy, nz + 2)
+    float* out_x;
+    float* out_y;
+    int nx, ny, nz, gx, gy, begin;  // grid (gx, gy, nz + 2)
 };
 struct BeamJob {     // beam-staged Siddon projection of one view list
     const float* stage_x;
@@ -352,7 +352,7 @@ int launch_residual_multi(const ResidualJob* d_jobs, int njobs, long long blocks
 int launch_quad_multi(const QuadJob* d_jobs, int njobs, long long blocks, hipStream_t stream);
 int launch_atb_multi(const AtbJob* d_jobs, int njobs, long long blocks, int zper, hipStream_t stream);
 // Block counts of one job of each kind (host side).
-int stage_job_blocks(const HostGeometry& g, int principal, int* gx, int* gy);
+int stage_job_blocks(const HostGeometry& g, int* gx, int* gy);
 long long beam_job_blocks(const HostGeometry& g, int ngroups, const BeamShape& shape);
 int residual_job_blocks(long long n);
 int quad_job_blocks(int nU, int nV, int nviews);

@@ -154,8 +154,8 @@ int ax_launch(const void* d_img, int dtype, const HostGeometry& g, const Forward
         if (!rec.stage_used[a]) continue;
         stage[a] = reinterpret_cast<float*>(ws);
         ws += align256((size_t)stage_elements(g, a) * sizeof(float));
-        TIGRE_CHECK(launch_stage_volume(d_img, dtype, g, a, stage[a], stream));
     }
+    if (rec.ngroups() > 0) TIGRE_CHECK(launch_stage_volume(d_img, dtype, g, stage, stream));
     if (rec.ngroups() > 0)
         TIGRE_CHECK(launch_ax_beam(stage[0], stage[1], g, d_views, d_groups, rec.ngroups(), rec.shape,
                                    projection_type, layout, d_proj, max_planes, stream));

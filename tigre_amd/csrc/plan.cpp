@@ -329,17 +329,18 @@ int tigre_batch_create(const TigreBatchStep* steps, int nsteps, TigreBatch* out)
         for (int a = 0; a < 2; ++a) {
             if (!rec.stage_used[a]) continue;
             stg[a] = reinterpret_cast<float*>(ws + stage_offset(g, rec, a));
+        }
+        if (rec.ngroups() > 0) {
             StageJob j;
             j.vol = st.d_x;
-            j.out = stg[a];
+            j.out_x = stg[0];
+            j.out_y = stg[1];
             j.nx = g.nVoxel[0];
             j.ny = g.nVoxel[1];
             j.nz = g.nVoxel[2];
-            j.principal = a;
-            j.na_pad = (a == 0 ? (g.nVoxel[1] + 3) & ~3 : (g.nVoxel[0] + 3) & ~3);
             j.begin = (int)b_stage;
-            b_stage += stage_job_blocks(g, a, &j.gx, &j.gy);
-            TIGRE_REQUIRE(j.gy <= 65535 && g.nVoxel[2] + 2 <= 65535, "volume too large for the staging copy");
+            b_stage += stage_job_blocks(g, &j.gx, &j.gy);
+            TIGRE_REQUIRE(g.nVoxel[2] + 2 <= 65535, "volume too large for the staging copy");
             stage.push_back(j);
         }
         if (rec.ngroups() > 0) {
