@@ -137,8 +137,9 @@ __device__ __forceinline__ void n_field(const float (&c)[kB], const float (&belo
 //
 // What bounds it: vector issue, 20 evaluations of n (a square root and a reciprocal each) for 8 stored rows a plane
 // with 3 wavefronts a SIMD; the halo costs 1.5 to 1.9 times the voxels.  20 iterations, two passes and a one-workgroup
-// sum an iteration before and this: 40 x 36 x 42 486 -> 151 us, 128^3 512 -> 363, 190 x 205 x 181 768 -> 528,
-// 256^3 970 -> 960 (its 256 columns fill 5 tiles of 60 badly); PICCS 134 x 157 x 133, 10 iterations, 480 -> 313.
+// sum an iteration with barriers and LDS before and this: 40 x 36 x 42 486 -> 151 us, 128^3 521 -> 361, 200^3 768 -> 578,
+// 256^3 975 -> 940 (its 256 columns fill 5 tiles of 60 badly), 400^3 4514 -> 3069, 512^3 7474 -> 6297; AwTV 240^3
+// 1164 -> 1092; PICCS 300^3 3216 -> 2396.
 template <int kKind, int kCore, bool kUpdate, bool kNorm>
 __global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(const float* __restrict__ f, float* __restrict__ out,
                                                         TvParams tp, int nx, int ny, int nz, int ntx, int nty,
@@ -252,6 +253,7 @@ __global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(cons
         };
         // the passes' planes: p reads f, p - 1 is updated, p - 2 adds to the norm
         constexpr int kLead = kUpdate && kNorm ? 1 : 0;
+        constexpr int kLow = kNorm ? 1 : 2;  // rows from which the updated image is formed
         const int begin = z0 - kLead, end = z1 + kLead;
         auto step = [&](int p, float (&v)[NF][kR]) {
             float u[kR];  // the image whose norm is taken, plane q
@@ -263,7 +265,7 @@ __global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(cons
             }
             if (kUpdate) {
                 const float alpha_p = p >= 1 && p <= nz ? scale : 0.0f;  // the zero slices stay 0
-                differences(p, Int<1>{}, Int<kR - 1>{}, cu, cu2, fp, pp, [&](int r, float val, float by, bool rest) {
+                differences(p, Int<kLow>{}, Int<kR - kLow>{}, cu, cu2, fp, pp, [&](int r, float val, float by, bool rest) {
                     if (rest) {
                         sp[r] = val;
                     } else {
@@ -271,7 +273,7 @@ __global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(cons
                     }
                 });
 #pragma unroll
-                for (int r = 1; r < kR - 1; ++r) formed(sp[r]);
+                for (int r = kLow; r < kR - kLow; ++r) formed(sp[r]);
                 if (kNorm) {  // copies of the edge voxels beyond the edges, as the loads give them
                     if (low_y) u[1] = u[2];
                     if (high_y) {
@@ -372,6 +374,28 @@ __global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(cons
 }
 
 namespace {
+long long ceil_div(long long a, long long b) { return (a + b - 1) / b; }
+
+// Planes of a chunk for `column` tiles a chunk of planes, each with `halo` planes beyond its own.  A CU takes one
+// workgroup of four tiles after another, and up to four at a time in about that multiple of the time of one (one or two
+// leave it waiting for its own loads and chains: 1.4 and 1.08); the chunks that cost a CU the least
+// are taken.  Measured, us for 20 iterations (tiles): 320^3 1654 (2880), 1672 (1920), 1808 (2400), 1917 (3120); 400^3
+// 3121 (2800), 3387 (1750), 3789 (3150); 512^3 6315 (4032), 6422 (2880), 6908 (1728), 9767 (4608).
+int tv_chunk(long long column, long long nz, int halo) {
+    int chunk = (int)nz;
+    double best = INFINITY;
+    for (long long chunks = 1; chunks <= std::max(1LL, nz / 4); ++chunks) {
+        const long long planes = ceil_div(nz, chunks), groups = ceil_div(column * ceil_div(nz, planes), kTvWaves);
+        const long long each = groups <= kTvBlocks ? ceil_div(groups, 256) : 4 * ceil_div(groups, kTvBlocks);
+        const double cost = (double)(each * (planes + halo)) * (each == 1 ? 1.4 : (each == 2 ? 1.08 : 1.0));
+        if (cost < best) {
+            best = cost;
+            chunk = (int)planes;
+        }
+    }
+    return chunk;
+}
+
 template <int kKind>
 int run_tv_descent(const float* img, float* dst, float alpha, const TvParams& tp, double norm_eps, long nx, long ny,
                    long nz, int maxiter, hipStream_t stream) {
@@ -386,13 +410,19 @@ int run_tv_descent(const float* img, float* dst, float alpha, const TvParams& tp
     const long long ntx = nx <= 63 ? 1 : (nx - 63 + kTvColumns - 1) / kTvColumns + 1;
     // 8 rows a tile cost the least halo; 2 rows and chunks from 2 planes give a small volume more wavefronts and
     // shorter ones (20 iterations: 40 x 36 x 42 151 us, 240 with 8 rows; 64^3 180 and 237; 128^3, 1536 tiles of 8
-    // rows, 383 and 363).  Chunks are as long as one round of the chip's slots allows (3 wavefronts a SIMD, 2 for
-    // PICCS; 256^3: 992 us with 3072 tiles, 1139 with 1536, 1145 with 4096).
+    // rows, 383 and 363).
     const bool small = ntx * ((ny + 7) / 8) * ((nz + 3) / 4) < 1024;
     const int rows = small ? 2 : 8;
-    const long long nty = (ny + rows - 1) / rows, slots = kKind == 2 && !small ? 2048 : 3072;
-    const int chunk = (int)std::min(64LL, std::max(small ? 2LL : 4LL, (nz * ntx * nty + slots - 1) / slots));
-    const long long ntiles = ntx * nty * ((nz + chunk - 1) / chunk);
+    const long long nty = (ny + rows - 1) / rows, column = ntx * nty;
+    // A pass that takes the norm too evaluates n on 20 rows for 8 and 4 planes more a chunk, a pass for each on 18 and 2,
+    // and moves 8 bytes a voxel instead of 12.  Two passes pay while the Infinity Cache serves them (us for 20
+    // iterations, one and two passes: TV 150 x 140 x 160 415 and 374, 200^3 587 and 578, 320^3 1578 and 1650, 512^3 6297
+    // and 8112; PICCS 200^3 1030 and 950, 300^3 2510 and 2396, 400^3 5775 and 6643), and always for AwTV, which
+    // spends most on the weights' exponentials (240 x 230 x 250 1374 and 1092).
+    const bool fused = small || (kKind == 0 && n > (1u << 23)) || (kKind == 2 && n > (1u << 25));
+    const int chunk = small ? (int)std::max(2LL, ceil_div(nz, std::max(1LL, 3072 / column)))
+                            : tv_chunk(column, nz, fused ? 4 : 2);
+    const long long ntiles = column * ((nz + chunk - 1) / chunk);
     TIGRE_REQUIRE(ntiles < (1LL << 30), "image too large");
     const int nblocks = (int)std::min((long long)kTvBlocks, (ntiles + kTvWaves - 1) / kTvWaves);
     StreamScratch scratch(stream);
@@ -417,8 +447,8 @@ int run_tv_descent(const float* img, float* dst, float alpha, const TvParams& tp
         if (rows == 8) TIGRE_TV(8, U, N); \
         else TIGRE_TV(2, U, N);         \
     } while (0)
-        if (it == 0) TIGRE_TV_ROWS(false, true);
-        if (last) TIGRE_TV_ROWS(true, false);
+        if (it == 0 || !fused) TIGRE_TV_ROWS(false, true);
+        if (last || !fused) TIGRE_TV_ROWS(true, false);
         else TIGRE_TV_ROWS(true, true);
 #undef TIGRE_TV_ROWS
 #undef TIGRE_TV
