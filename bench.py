@@ -833,7 +833,7 @@ def bench_tv(args):
         log("TV %d^3: %.1f us per iteration, 20 iterations %.3f ms" % (n, it_ms * 1e3, call_ms))
         del img
         torch.cuda.empty_cache()
-    result = {"metric": "minimizeTV iteration time (two passes + norm)", "value": out["512^3"]["iteration_us"],
+    result = {"metric": "minimizeTV iteration time (step and norm)", "value": out["512^3"]["iteration_us"],
               "unit": "us per iteration at 512^3", "n_gpus": 1, "steps": args.steps, "warmup": 1,
               "higher_is_better": False, "dtype": "f32", "data": "synthetic (seeded 40-ellipsoid phantoms)",
               "config": {"workload": "minTV 20 iterations at 256^3 and 512^3"}, "by_size": out}
