@@ -384,7 +384,8 @@ long long ceil_div(long long a, long long b) { return (a + b - 1) / b; }
 int tv_chunk(long long column, long long nz, int halo) {
     int chunk = (int)nz;
     double best = INFINITY;
-    for (long long chunks = 1; chunks <= std::max(1LL, nz / 4); ++chunks) {
+    for (int most = 1; most <= 64; most += most < 4 ? 1 : 4) {  // workgroups a CU: as many chunks as that allows
+        const long long chunks = std::max(1LL, std::min(256LL * kTvWaves * most / column, nz / 4));
         const long long planes = ceil_div(nz, chunks), groups = ceil_div(column * ceil_div(nz, planes), kTvWaves);
         const long long each = groups <= kTvBlocks ? ceil_div(groups, 256) : 4 * ceil_div(groups, kTvBlocks);
         const double cost = (double)(each * (planes + halo)) * (each == 1 ? 1.4 : (each == 2 ? 1.08 : 1.0));
