@@ -566,7 +566,7 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
         __syncthreads();
         na = __builtin_amdgcn_readfirstlane(sh.ext[0]);
         nzb = __builtin_amdgcn_readfirstlane(sh.ext[1]);
-        if (na * nzb * (pl_try + tap) <= kSlabCap) {
+        if (na * nzb * (pl_try + tap) <= kSlabCap && slab_offsets_fit(pl_try + tap, nzb, sg.NZ, sg.NA)) {
             staged = true;
             planes = pl_try;
             first_slab = __builtin_amdgcn_readfirstlane(sh.live[0]);
@@ -580,7 +580,7 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
     const int SP = kMode == 0 ? kSlabCap / max(planes, 1) : nzb * na;
     const bool down = kMode == 0 && dir < 0;  // the first LDS plane is the highest
     // this thread's quads of a box: row (plane, z) and 4-float column, as a byte offset from the box's lowest
-    // corner (32 bits: a box spans few planes); quads in the pad between planes and after the last copy the corner
+    // corner (32 bits: slab_offsets_fit); quads in the pad between planes and after the last copy the corner
     const int nq4 = max(na >> 2, 1), prow = max(kMode == 0 ? SP >> 2 : nzb * nq4, 1);  // row and plane in quads
     const int nq = (planes + tap) * prow;                                             // of a full slab
     constexpr int kLoads = (kSlabCap / 4 + kBeamThreads - 1) / kBeamThreads;
@@ -591,7 +591,8 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
         const int pl = q / prow, rest = q - pl * prow;
         const int zr = rest / nq4, aq = rest - zr * nq4;
         const bool in = pl < planes + tap && zr < nzb;
-        qoff[j] = in ? 4u * (unsigned)(((down ? planes - 1 - pl : pl) * sg.NZ + zr) * sg.NA + 4 * aq) : 0u;
+        const unsigned row = (unsigned)(down ? planes - 1 - pl : pl) * (unsigned)sg.NZ + (unsigned)zr;
+        qoff[j] = in ? 4u * (row * (unsigned)sg.NA + 4u * (unsigned)aq) : 0u;
     }
     // the slabs' table, one slab per lane (a short last slab's lowest corner is where a full one's would be)
     const int cells_total = last_cell + 2;

@@ -218,6 +218,13 @@ int launch_ax_siddon(const float* bricked, const HostGeometry& g, const BrickGri
 // (0 = x, 1 = y): [p][z][a] with a zero border, a = the other horizontal axis.
 long long stage_elements(const HostGeometry& g, int principal);
 int launch_stage_volume(const void* vol, int dtype, const HostGeometry& g, float* const* stage, hipStream_t stream);
+// Whether the byte offsets of the beam kernel's copies of `planes` consecutive planes (rows of a box of `rows` rows; a
+// plane of the staging copy has stage_rows x stage_columns floats) stay below 2^31.  The kernel forms them in 32 bits;
+// a volume thin along the rays has planes of which few fit (13000 x 13000: four).
+__host__ __device__ inline bool slab_offsets_fit(int planes, int rows, int stage_rows, int stage_columns) {
+    const unsigned long long last = (unsigned long long)(planes - 1) * (unsigned)stage_rows + (unsigned)rows;
+    return last * (unsigned)stage_columns <= (1ull << 29);
+}
 // The rays of a beam workgroup: a tile of units_u x units_v units of 16 x 4 pixels in each of
 // 16 / (units_u units_v) views.
 struct BeamShape {
