@@ -283,6 +283,8 @@ __device__ __forceinline__ int plane_range(const PlaneRay& r, int first, int cou
 // Cells first .. first + count - 1 of the sweep (at most eight); the ray's voxel is at r.off + slot of
 // `base`, planes PS apart (kPS > 0: this constant).  kRim: a ray of the tile may lie outside the volume
 // here; outside, it stays on the border, whose voxels are 0, and enters with the index that the border is next to.
+// kLds: from LDS, where a term of no length is added as 0 v; else from the staging copy, where it is left out (an
+// infinite or undefined voxel makes the one NaN, not the other).
 template <bool kLds, int kPS, bool kRim>
 __device__ __forceinline__ void plane_cells(PlaneRay& r, const float* __restrict__ base, unsigned slot, unsigned PS,
                                             int nA, int nz, int first, int count) {
@@ -315,9 +317,12 @@ __device__ __forceinline__ void plane_cells(PlaneRay& r, const float* __restrict
         const unsigned stepA = cA ? dA : 0u, stepz = cz ? dZ : 0u;
         const unsigned mid = off + (tA < tz ? stepA : stepz), end = off + stepA + stepz;
         const float t1 = fminf(tA, tz), t2 = fmaxf(tA, tz);
-        sum = fmaf(t1, read(off), sum);
-        sum = fmaf(t2 - t1, read(mid), sum);
-        sum = fmaf(1.0f - t2, read(end), sum);
+        auto add = [&](float t, unsigned o) {
+            if (kLds || t != 0.0f) sum = fmaf(t, read(o), sum);
+        };
+        add(t1, off);
+        add(t2 - t1, mid);
+        add(1.0f - t2, end);
         off = kPS > 0 ? end : end + (PS << kSh);
     }
     r.off = (off >> kSh) - slot;
@@ -359,6 +364,7 @@ struct SweepShared {
     int4 box[kMaxSlabs];     // per slab, see SlabBox (during planning: a0, z0, rim)
     int ext[2];              // box extents na (multiple of 4) and nzb, maxed over the slabs
     int live[2];             // first and last slab whose box meets the volume (Siddon)
+    int again[4];            // staging copy's rows and columns, direction, planes: for the rays that are walked again
 };
 
 // Per-ray state of the interpolated projector (ray_interpolated_projection.cu
@@ -535,6 +541,7 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
     // box fits an LDS buffer ----
     int planes = 0, first_slab = 0, nslabs = 0, na = 0, nzb = 0;
     bool staged = false;
+    if (kMode == 0 && tid == 0) sh.again[0] = sg.NZ, sh.again[1] = sg.NA, sh.again[2] = dir, sh.again[3] = nP;
     for (int attempt = 0; attempt < 5 && !staged; ++attempt) {
         int pl_try = attempt == 0 ? max_planes
                                   : min(max_planes, attempt == 1 ? 6 : (attempt == 2 ? 4 : (attempt == 3 ? 2 : 1)));
@@ -682,15 +689,7 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
             r.sum = r.part = 0.0f;
             plane_axis(sp[1 - kP], kP == 0 ? ry : rx, a0, da, nA, r.A0, r.kA, r.iA, r.dA);
             plane_axis(sp[2], rz, a0, da, nz, r.z0, r.kz, r.iz, r.dZ);
-            if (!staged) {
-                // the beam's box does not fit an LDS buffer: read the staging copy
-                r.off = plane_offset(r, 0, 0, 0, sg.NA, nA, nz) + (unsigned)stage_index(sg, dir > 0 ? -1 : nP, 0, 0);
-                r.dZ *= sg.NA;
-                if (active)
-                    for (int c = 0; c < nP + 2; c += 8)
-                        plane_cells<false, 0, true>(r, stage, 0u, (unsigned)(dir * sg.NZ * sg.NA), nA, nz, c,
-                                                    min(8, nP + 2 - c));
-            } else {
+            if (staged) {
                 r.dZ *= na;
                 int at0 = 0;         // origin offset of the box that r.off refers to
                 bool carry = false;  // r.off is the ray's voxel
@@ -720,6 +719,20 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
                     else
                         plane_cells<true, kPlaneStride, false>(r, sh.buf, at, 0u, nA, nz, first, 8);
                 });
+            }
+            // A beam whose box does not fit an LDS buffer reads the staging copy; so does a ray whose sum is not a
+            // number, once more, without the terms of no length.
+            const float swept = r.sum + r.part;
+            if (active && (!staged || swept != swept)) {
+                // from LDS: uniform values kept for this through the sweep cost it 1 % (they spilled)
+                const StageGeom g2{sh.again[0], sh.again[1]};
+                const int dir2 = sh.again[2], nP2 = sh.again[3];
+                r.sum = r.part = 0.0f;
+                r.dZ = r.dZ > 0 ? g2.NA : -g2.NA;
+                r.off = plane_offset(r, 0, 0, 0, g2.NA, nA, nz) + (unsigned)stage_index(g2, dir2 > 0 ? -1 : nP2, 0, 0);
+                for (int c = 0; c < nP2 + 2; c += 8)
+                    plane_cells<false, 0, true>(r, stage, 0u, (unsigned)(dir2 * g2.NZ * g2.NA), nA, nz, c,
+                                                min(8, nP2 + 2 - c));
             }
             store((double)(r.sum + r.part) * (len * da));  // the sum is in cells
             return;
