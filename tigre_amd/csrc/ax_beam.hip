@@ -209,23 +209,27 @@ __device__ inline bool walk(RayWalk& r, const float* __restrict__ base, unsigned
 // below 1), so a cell holds at most two crossings and three segments.  A and z are taken in mirrored
 // indices that increase along the sweep and in fixed point with 32 fraction bits, A(s) = A0 + s kA, s counted in
 // cells from cell -1.  In the cell the ray enters at fraction f of an A voxel it crosses the next A plane
-// at the fraction tA = min((1 - f) / kA, 1) of the cell, and likewise in z.  With t1 <= t2 the two
+// at the fraction tA = min((1 - f) / kA, 1) of the cell, and likewise in z; 1 - f is what the cell carries (rounded to
+// FP32 near 1, f would lose a crossing that is near: 2^-24 voxel, a whole cell at a slope of 6e-8).  With t1 <= t2 the two
 // sorted, the cell adds
 //     t1 v0 + (t2 - t1) v1 + (1 - t2) v2,
 // v0 the entry voxel, v1 the one past the first crossing, v2 the exit voxel.  Whether an axis crosses is the
-// carry of the fraction's addition, so voxel and position cannot part, a voxel that is not crossed is
+// borrow of the rest's subtraction, so voxel and position cannot part, a voxel that is not crossed is
 // not read.  The cells of each eight are summed by themselves first: adding the same voxel value again and again
 // rounds the same way each time, and one sum over 1024 cells was off by 2.6e-6 on a phantom of constant regions
 // (rel-L2 at 1024^3; 3.7e-7 in eights).  Slabs have 8, 4, 2 or 1 cells and start at multiples of that, so the sums do not
 // depend on how a sweep is cut.  The slope in 32 bits puts a ray
-// at most 2^-33 voxel a cell off its line (1e-7 after 1024 cells); an FP32 crossing time is
-// off by 3e-5 voxel there.
+// at most 2^-33 voxel a cell off its line (1e-7 after 1024 cells), which moves a crossing by that over the slope; an FP32
+// crossing time is off by 3e-5 cells there.  Rays with a smaller slope than flat_slope() on an axis that they move on
+// therefore take the crossing walk.  Off by, here and there (rms over rays that cross one plane, random voxels): 64
+// cells, slope 2^-12: 1.5e-7, 1.7e-7; 256, 2^-13: 2.7e-7, 3.0e-7; 1024, 2^-14: 5.4e-7, 7.1e-7; 64, 2^-14: 5.9e-7, 1.8e-7.
 //
 // The step has no branch and no division, about 20 VALU instructions and (planes at a constant LDS stride, so
 // the plane is an immediate of the read) three LDS reads, all lanes in step; the crossing walk above takes
 // one crossing per step, about 17 instructions each, 1.6 times a cell on average, and its lanes leave a slab
 // at different steps.  It stays for rays with a slope of 1 or more (detector tiles that look across the 45
-// degree diagonal, about 4 % of them at a fan angle of 15 degrees).
+// degree diagonal, about 4 % of them at a fan angle of 15 degrees) and for the flat ones (a pixel row or column about
+// the central one, where pixels are smaller than about 2^-12 of the source's distance).
 //
 // Measured at 512^3 voxels, 512^2 pixels, 360 views: 25.3 ms, 36.5 ms with the crossing walk alone; 23 VALU
 // instructions per ray and plane (33.8 before), 3.4 cycles each (most pairs of an FMA and another operation
@@ -235,11 +239,15 @@ __device__ inline bool walk(RayWalk& r, const float* __restrict__ base, unsigned
 struct PlaneRay {
     unsigned long long A0, z0;  // mirrored A and z at the start of cell -1, 2^-32 voxel
     unsigned kA, kz;            // slopes, 2^-32 voxel
-    float iA, iz;               // their reciprocals
+    float iA, iz;               // their reciprocals, in cells per 2^-32 voxel
     int dA, dZ;                 // offset step of one (mirrored) index on A (1 or -1) and on z (row steps)
     unsigned off;               // voxel offset in the current source, as in RayWalk
     float sum, part;            // of the whole eights of cells so far, of the cells since
 };
+
+// Smallest slope of the plane walk over nP planes: where it is as exact as the crossing walk, whose times round to
+// nP 2^-24 cells.
+__device__ __forceinline__ float flat_slope(int nP) { return fmaxf(0x1p-9f / sqrtf((float)nP), 0x1p-6f / (float)nP); }
 
 // Mirrored position and slope on one axis of the line s0 + r a, from the start of cell -1, which the
 // sweep enters at parameter a0 and leaves da later; a ray parallel to the axis stays inside its voxel
@@ -257,7 +265,7 @@ __device__ __forceinline__ void plane_axis(double s0, double r, double a0, doubl
     const double f = floor(x);
     x0 = ((unsigned long long)(long long)f << 32) + (unsigned long long)((x - f) * 4294967296.0);
     k = (unsigned)rint(slope * 4294967296.0);
-    ik = k != 0u ? (float)(1.0 / slope) : 1e30f;
+    ik = k != 0u ? (float)(0x1p-32 / slope) : 1e20f;
 }
 
 // Offset of the voxel of a ray at the start of cell `first`, in a box of origin (a0, z0) and row length na;
@@ -291,11 +299,10 @@ __device__ __forceinline__ void plane_cells(PlaneRay& r, const float* __restrict
     constexpr int kSh = kLds ? 2 : 0;  // byte offsets in LDS, element offsets in the staging copy
     const unsigned long long xA = r.A0 + (unsigned long long)r.kA * (unsigned)first;
     const unsigned long long xz = r.z0 + (unsigned long long)r.kz * (unsigned)first;
-    unsigned A = (unsigned)xA, z = (unsigned)xz;
+    unsigned A = ~(unsigned)xA, z = ~(unsigned)xz;  // what is left to the next plane
     int iA = (int)(xA >> 32), iz = (int)(xz >> 32);
     const unsigned dA = (unsigned)r.dA << kSh, dZ = (unsigned)r.dZ << kSh;
     unsigned off = (r.off + slot) << kSh;
-    const float sA = r.iA * 0x1p-32f, sz = r.iz * 0x1p-32f;
     float sum = kPS > 0 ? 0.0f : r.part;  // a constant stride: eight cells
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -304,9 +311,9 @@ __device__ __forceinline__ void plane_cells(PlaneRay& r, const float* __restrict
             return kLds ? *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (o + (kPS > 0 ? 4 * kPS * j : 0)))
                         : base[o];
         };
-        const float tA = __builtin_amdgcn_fmed3f(fmaf((float)A, -sA, r.iA), 0.0f, 1.0f);
-        const float tz = __builtin_amdgcn_fmed3f(fmaf((float)z, -sz, r.iz), 0.0f, 1.0f);
-        bool cA = __builtin_add_overflow(A, r.kA, &A), cz = __builtin_add_overflow(z, r.kz, &z);
+        const float tA = __builtin_amdgcn_fmed3f((float)A * r.iA, 0.0f, 1.0f);
+        const float tz = __builtin_amdgcn_fmed3f((float)z * r.iz, 0.0f, 1.0f);
+        bool cA = __builtin_sub_overflow(A, r.kA, &A), cz = __builtin_sub_overflow(z, r.kz, &z);
         if (kRim) {
             const bool inA = (unsigned)(iA + 1) <= (unsigned)nA, inz = (unsigned)(iz + 1) <= (unsigned)nz;
             iA += cA ? 1 : 0;
@@ -667,22 +674,23 @@ __device__ inline void beam_sweep(const float* __restrict__ stage, const StageGe
     double rz = ray_dir(w, u, pv, 2);
     if (kMode == 0) {
         // The plane walk, unless a ray of the 16 x 16 pixels around this unit has a slope of 1 or more in
-        // its view (their corner rays hold the extremes: the slopes are linear-fractional in the pixel).
+        // its view (their corner rays hold the extremes: the slopes are linear-fractional in the pixel), or one of the
+        // unit's own a slope below flat_slope().
         // This depends on the pixel and the view alone, so a ray's sum does not depend on the group.
-        bool steep;
-        {
-            const int cu = min((u & ~15) + ((lane & 1) ? 15 : 0), nU - 1);
-            const double cv = (double)(nV - 1 - min((v & ~15) + ((lane & 2) ? 15 : 0), nV - 1));
-            const double dP = 0.999 * fabs(ray_dir(w, cu, cv, kP));
-            steep = __ballot(!(fabs(ray_dir(w, cu, cv, 1 - kP)) < dP && fabs(ray_dir(w, cu, cv, 2)) < dP)) != 0;
-        }
+        const int cu = min((u & ~15) + ((lane & 1) ? 15 : 0), nU - 1);
+        const double cv = (double)(nV - 1 - min((v & ~15) + ((lane & 2) ? 15 : 0), nV - 1));
+        const double dP = 0.999 * fabs(ray_dir(w, cu, cv, kP));
+        const bool steep = !(fabs(ray_dir(w, cu, cv, 1 - kP)) < dP && fabs(ray_dir(w, cu, cv, 2)) < dP);
         if (w.pad[1] != 0.0) parallel_siddon_height(sp, rx, ry, rz, nx, ny);
         // components below 1e-3 voxel are treated as exactly zero (:155-159)
         if (fabs(rx) < 1e-3) rx = 0.0;
         if (fabs(ry) < 1e-3) ry = 0.0;
         if (fabs(rz) < 1e-3) rz = 0.0;
+        const float flat = flat_slope(nP) * fabsf((float)(kP == 0 ? rx : ry));
+        const float ra = fabsf((float)(kP == 0 ? ry : rx)), rh = fabsf((float)rz);
+        const bool crossings = __ballot(steep || (active && ((ra > 0.0f && ra < flat) || (rh > 0.0f && rh < flat)))) != 0;
         const double len = sqrt(rx * rx * dvx * dvx + ry * ry * dvy * dvy + rz * rz * dvz * dvz);  // mm (:241, :267)
-        if (!steep) {  // uniform per wavefront; both branches pass the same barriers
+        if (!crossings) {  // uniform per wavefront; both branches pass the same barriers
             const double rp = kP == 0 ? rx : ry;
             const double da = 1.0 / fabs(rp), a0 = ((dir > 0 ? -1.0 : (double)nP + 1.0) - sp[kP]) / rp;
             PlaneRay r;
