@@ -383,22 +383,28 @@ struct RaySamples {
     float sum;
 };
 
+// Product of a box-relative index and a stride: both below 2^24 in an LDS box; a plane of the staging copy can be larger.
+template <bool kLds>
+__device__ __forceinline__ unsigned stride_mul(unsigned i, unsigned stride) {
+    return kLds ? __umul24(i, stride) : i * stride;
+}
+
 // Trilinear (kMode 1) or nearest (kMode 2) sample of a box whose fastest axis
 // is A: `src` holds planes P, rows z, columns A with strides SP and SZ; (pc, zc,
 // ac) is the lower tap relative to the box origin.
-template <int kMode>
+template <int kMode, bool kLds>
 __device__ __forceinline__ float box_sample(const float* __restrict__ src, int SP, int SZ, float P, float A, float Z,
                                             int P0, int Z0, int A0) {
-    // tap indices relative to the box origin are >= 0 and < 2^24, strides < 2^24
+    // tap indices relative to the box origin are >= 0
     if (kMode == 2) {
         const unsigned pc = (unsigned)((int)floorf(P + 0.5f) - P0), zc = (unsigned)((int)floorf(Z + 0.5f) - Z0),
                        ac = (unsigned)((int)floorf(A + 0.5f) - A0);
-        return src[__umul24(pc, (unsigned)SP) + __umul24(zc, (unsigned)SZ) + ac];
+        return src[stride_mul<kLds>(pc, (unsigned)SP) + stride_mul<kLds>(zc, (unsigned)SZ) + ac];
     }
     const float flP = floorf(P), flA = floorf(A), flZ = floorf(Z);
     const float wP = P - flP, wA = A - flA, wZ = Z - flZ;
-    const unsigned o = __umul24((unsigned)((int)flP - P0), (unsigned)SP) +
-                       __umul24((unsigned)((int)flZ - Z0), (unsigned)SZ) + (unsigned)((int)flA - A0);
+    const unsigned o = stride_mul<kLds>((unsigned)((int)flP - P0), (unsigned)SP) +
+                       stride_mul<kLds>((unsigned)((int)flZ - Z0), (unsigned)SZ) + (unsigned)((int)flA - A0);
     const float c00 = fmaf(wA, src[o + 1] - src[o], src[o]);
     const float c10 = fmaf(wA, src[o + SZ + 1] - src[o + SZ], src[o + SZ]);
     const float c01 = fmaf(wA, src[o + SP + 1] - src[o + SP], src[o + SP]);
@@ -462,14 +468,14 @@ __device__ inline bool sample_slab(RaySamples& r, const float* __restrict__ base
         const float A = __builtin_amdgcn_fmed3f(fmaf(fm, fA, qA), -1.0f, hA);
         const float Z = __builtin_amdgcn_fmed3f(fmaf(fm, fz, qz), -1.0f, hz);
         if (kMode == 2) {
-            sum += box_sample<kMode>(base + slot, SP, SZ, P, A, Z, P0, Z0, A0);
+            sum += box_sample<kMode, kLds>(base + slot, SP, SZ, P, A, Z, P0, Z0, A0);
         } else {
             const float flP = floorf(P), flA = floorf(A), flZ = floorf(Z);
             const float wP = P - flP, wA = A - flA, wZ = Z - flZ;
             const unsigned o =
                 kLds ? (unsigned)fmaf(flP - fP0, fSP, fmaf(flZ, fSZ, flA - cza))
-                     : __umul24((unsigned)((int)flP - P0), (unsigned)SP) +
-                           __umul24((unsigned)((int)flZ - Z0), (unsigned)SZ) + (unsigned)((int)flA - A0);
+                     : stride_mul<kLds>((unsigned)((int)flP - P0), (unsigned)SP) +
+                           stride_mul<kLds>((unsigned)((int)flZ - Z0), (unsigned)SZ) + (unsigned)((int)flA - A0);
             if (o != cached) {
                 const float* t = base + o;
                 c000 = t[0];
