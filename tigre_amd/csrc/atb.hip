@@ -221,33 +221,34 @@ constexpr int kBatch = 4;
 constexpr int kStrip = 8;
 }  // namespace
 
-// kN quads of one column from row position pv on and their v weights, from a
-// staged window (LDS) or from the quad copy in global memory.  kClamp: the
+// kN quads of one column at row positions pv + z dpv, z = z0, z0 + 1, ..., and
+// their v weights, from a staged window (LDS) or from the quad copy in global
+// memory.  The positions are rounded once each: added up slice by slice, 31
+// roundings at a row number of 1000 are 1e-4 pixel.  kClamp: the
 // column may leave the detector's rows.  The LDS pointer is
 // restrict-qualified: its reads then carry alias-scope information, and the
 // compiler does not make them wait for the direct LDS loads of the next view
 // (into the other window) that are still in flight.
 template <int kN, bool kClamp>
-__device__ __forceinline__ void read_lds(const char* __restrict__ lds, int lb, float& pv, float dpv, float lo, float hi,
-                                         float4 (&q)[kN], float (&wv)[kN]) {
+__device__ __forceinline__ void read_lds(const char* __restrict__ lds, int lb, float pv, float dpv, float z0, float lo,
+                                         float hi, float4 (&q)[kN], float (&wv)[kN]) {
 #pragma unroll
     for (int k = 0; k < kN; ++k) {
-        const float at = kClamp ? __builtin_amdgcn_fmed3f(pv, lo, hi) : pv;
+        const float row = fmaf(z0 + (float)k, dpv, pv);
+        const float at = kClamp ? __builtin_amdgcn_fmed3f(row, lo, hi) : row;
         wv[k] = __builtin_amdgcn_fractf(at);
         q[k] = *reinterpret_cast<const float4*>(lds + ((int)((unsigned)at << 9) + lb));
-        pv += dpv;
     }
 }
 
 template <int kN>
-__device__ __forceinline__ void read_global(const char* pjb, unsigned rowb, unsigned colb, float& pv, float dpv,
-                                            float hv, float4 (&q)[kN], float (&wv)[kN]) {
+__device__ __forceinline__ void read_global(const char* pjb, unsigned rowb, unsigned colb, float pv, float dpv,
+                                            float z0, float hv, float4 (&q)[kN], float (&wv)[kN]) {
 #pragma unroll
     for (int k = 0; k < kN; ++k) {
-        const float at = __builtin_amdgcn_fmed3f(pv, 0.0f, hv);
+        const float at = __builtin_amdgcn_fmed3f(fmaf(z0 + (float)k, dpv, pv), 0.0f, hv);
         wv[k] = __builtin_amdgcn_fractf(at);
         q[k] = *reinterpret_cast<const float4*>(pjb + (__umul24((unsigned)at, rowb) + colb));
-        pv += dpv;
     }
 }
 
@@ -424,13 +425,12 @@ __device__ __forceinline__ void atb_lds_block(const float* __restrict__ proj, in
             fetch(p + 1, offset, blocks, row);
             const ViewParams v = next;
             next = view_params(views[min(p + 2, nviews - 1)]);
-            float pv = nb > 0 ? c.pv0 - r0 : c.pv0;
-            for (int z = za; z < z0; ++z) pv += c.dpv;
+            const float pv = nb > 0 ? c.pv0 - r0 : c.pv0;
 #pragma unroll
             for (int k = 0; k < kZ; k += kN) {
                 float4 q[kN];
                 float wv[kN];
-                read(lb, r0, pv, q, wv);
+                read(lb, r0, pv, (float)(z0 - za + k), q, wv);
                 __builtin_amdgcn_sched_barrier(0);
                 float wt[kN];
 #pragma unroll
@@ -456,16 +456,16 @@ __device__ __forceinline__ void atb_lds_block(const float* __restrict__ proj, in
         // runs of views of one kind: a branch within the view loop would move the sums between registers
         while (p < nviews) {
             while (p < nviews && blocks >= 32)
-                view([&](int lb, float, float& pv, float4 (&q)[kN], float (&wv)[kN]) {
-                    read_lds<kN, false>(lds, lb, pv, c.dpv, 0.0f, 0.0f, q, wv);
+                view([&](int lb, float, float pv, float z, float4 (&q)[kN], float (&wv)[kN]) {
+                    read_lds<kN, false>(lds, lb, pv, c.dpv, z, 0.0f, 0.0f, q, wv);
                 });
             while (p < nviews && blocks > 0 && blocks < 32)
-                view([&](int lb, float r0, float& pv, float4 (&q)[kN], float (&wv)[kN]) {
-                    read_lds<kN, true>(lds, lb, pv, c.dpv, -r0, hv - r0, q, wv);
+                view([&](int lb, float r0, float pv, float z, float4 (&q)[kN], float (&wv)[kN]) {
+                    read_lds<kN, true>(lds, lb, pv, c.dpv, z, -r0, hv - r0, q, wv);
                 });
             while (p < nviews && blocks == 0)
-                view([&](int, float, float& pv, float4 (&q)[kN], float (&wv)[kN]) {
-                    read_global<kN>(qbase + (long long)p * viewb, rowb, c.colb, pv, c.dpv, hv, q, wv);
+                view([&](int, float, float pv, float z, float4 (&q)[kN], float (&wv)[kN]) {
+                    read_global<kN>(qbase + (long long)p * viewb, rowb, c.colb, pv, c.dpv, z, hv, q, wv);
                 });
         }
     }
