@@ -157,9 +157,7 @@ int upload_async(void** d_ptr, const void* host, size_t bytes, size_t total, hip
 class StreamScratch {
   public:
     explicit StreamScratch(hipStream_t stream) : stream_(stream) {}
-    ~StreamScratch() {
-        for (void* p : blocks_) (void)hipFreeAsync(p, stream_);
-    }
+    ~StreamScratch() { release(); }
     StreamScratch(const StreamScratch&) = delete;
     StreamScratch& operator=(const StreamScratch&) = delete;
     template <typename T>
@@ -169,6 +167,19 @@ class StreamScratch {
         blocks_.push_back(q);
         *p = static_cast<T*>(q);
         return TIGRE_OK;
+    }
+    // alloc for a caller that can do with less: false, without an error left behind, when the block cannot be had.
+    template <typename T>
+    bool try_alloc(T** p, size_t bytes) {
+        if (alloc(p, bytes) == TIGRE_OK) return true;
+        (void)hipGetLastError();
+        set_error("");
+        return false;
+    }
+    // Gives the blocks back before the guard goes out of scope.
+    void release() {
+        for (void* p : blocks_) (void)hipFreeAsync(p, stream_);
+        blocks_.clear();
     }
     // A block of total bytes that starts with a copy of the host's bytes.
     int upload(void** p, const void* host, size_t bytes, size_t total) {
