@@ -57,8 +57,9 @@ class ViewSets:
     """Projector calls on fixed subsets of views of one geometry.
 
     The per-subset geometry (checked, rounded to float32, converted to the C
-    struct) is prepared once, when the subset is first used; ``ax``/``atb``
-    then call the device entry points directly on the current stream."""
+    struct) is prepared once, when the subset is first used, from the geometry
+    and indices as they were given; ``ax``/``atb`` then call the device entry
+    points directly on the current stream."""
 
     def __init__(self, geo, angles, blocks):
         self.geo = duplicate(geo)
@@ -67,7 +68,10 @@ class ViewSets:
         # the reference's Ax / Atb pick the parallel-beam operators from
         # geo.mode (_Ax.pyx:67-87, _Atb.pyx:56-76)
         self.parallel = getattr(self.geo, "mode", "cone") == "parallel"
-        self.blocks = [np.asarray(idx, dtype=np.int64).reshape(-1) for idx in blocks]
+        self.blocks = [np.array(idx, dtype=np.int64).reshape(-1) for idx in blocks]
+        for idx in self.blocks:
+            self.angles[idx]  # an index out of range is refused here
+        self._source = duplicate(self.geo), [idx.copy() for idx in self.blocks]
         self._sets = [None] * len(self.blocks)
         self.lib = _native.lib()
         self.vol_shape = tuple(int(v) for v in np.asarray(self.geo.nVoxel))
@@ -82,10 +86,15 @@ class ViewSets:
     def set(self, j):
         """(views, geometry, C geometry, float32 angles) of subset j."""
         if self._sets[j] is None:
-            idx = self.blocks[j]
-            g = prepared(_sub_geometry(self.geo, idx), self.angles[idx])
+            geo, idx = self._source[0], self._source[1][j]
+            g = prepared(_sub_geometry(geo, idx), geo.angles[idx])
             self._sets[j] = (idx, g, _native.CGeometry(g, len(idx)), np.ascontiguousarray(g.angles, dtype=np.float32))
         return self._sets[j]
+
+    @property
+    def sets(self):
+        """All subsets, as ``set`` gives them."""
+        return [self.set(j) for j in range(len(self))]
 
     def ax(self, img, j, kind=_native.PROJ_SIDDON, out=None):
         """Projections of subset j, stored like ``img`` (float32, bfloat16 or float16)."""
