@@ -246,7 +246,9 @@ def duplicate(geo):
     for attr, val in geo.__dict__.items():
         kind = type(val)
         if kind is np.ndarray and val.dtype.kind in "fiub":
-            new[attr] = val.copy(order="K")
+            if id(val) not in memo:  # an array that two fields share stays shared
+                memo[id(val)] = val.copy(order="K")
+            new[attr] = memo[id(val)]
         elif val is None or kind in (float, int, bool, str):
             new[attr] = val
         else:
