@@ -71,8 +71,12 @@ class ViewSets:
         self.blocks = [np.array(idx, dtype=np.int64).reshape(-1) for idx in blocks]
         for idx in self.blocks:
             self.angles[idx]  # an index out of range is refused here
-        self._source = duplicate(self.geo), [idx.copy() for idx in self.blocks]
         self._sets = [None] * len(self.blocks)
+        self._source = self.geo, self.blocks
+        if len(self.blocks) == 1:
+            self.set(0)
+        else:  # subsets may be many, and plans need none of them: their copies wait, those of what they are made from do not
+            self._source = duplicate(self.geo), [idx.copy() for idx in self.blocks]
         self.lib = _native.lib()
         self.vol_shape = tuple(int(v) for v in np.asarray(self.geo.nVoxel))
         self.det_shape = (int(self.geo.nDetector[0]), int(self.geo.nDetector[1]))

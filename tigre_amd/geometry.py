@@ -246,9 +246,10 @@ def duplicate(geo):
     for attr, val in geo.__dict__.items():
         kind = type(val)
         if kind is np.ndarray and val.dtype.kind in "fiub":
-            if id(val) not in memo:  # an array that two fields share stays shared
-                memo[id(val)] = val.copy(order="K")
-            new[attr] = memo[id(val)]
+            if id(val) in memo:  # an array that two fields share stays shared
+                new[attr] = memo[id(val)]
+            else:
+                new[attr] = memo[id(val)] = val.copy(order="K")
         elif val is None or kind in (float, int, bool, str):
             new[attr] = val
         else:
