@@ -66,14 +66,26 @@ def filtering(proj, geo, angles, parker=False, verbose=False):
     return weighted_filtering(proj, None, geo, angles)
 
 
-def _plain(t):
-    """A tensor whose memory a kernel may read behind autograd's and torch.func's back."""
+def _unwatched(t):
+    """A plain strided tensor that nothing follows: no recorded gradient, forward-mode tangent, torch.func transform,
+    trace, compilation or dispatch mode, all of which would miss a kernel that is not a torch operation."""
     import torch
 
-    return (type(t) is torch.Tensor and t.is_cuda and t.layout == torch.strided
-            and not (torch.is_grad_enabled() and t.requires_grad)
-            and torch.autograd.forward_ad._current_level < 0 and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and not t.is_neg())
+    if type(t) is not torch.Tensor or t.layout != torch.strided or (torch.is_grad_enabled() and t.requires_grad):
+        return False
+    if torch.jit.is_tracing() or torch.compiler.is_compiling():
+        return False
+    # private to torch: where one is missing, the general path is taken
+    wrapped = getattr(getattr(torch._C, "_functorch", None), "is_functorch_wrapped_tensor", None)
+    modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+    if wrapped is None or modes is None or wrapped(t) or modes() > 0:
+        return False
+    return torch.autograd.forward_ad.unpack_dual(t).tangent is None and not t.is_neg()
+
+
+def _plain(t):
+    """A tensor whose memory a kernel may read behind torch's back."""
+    return t.is_cuda and _unwatched(t)
 
 
 def weighted_filtering(proj, weight, geo, angles):
