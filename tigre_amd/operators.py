@@ -84,8 +84,10 @@ def _storage_code(t):
 def _stream_handle():
     import torch
 
-    if torch.cuda.is_initialized():  # the current stream without a Stream object around it
-        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    # the current stream without a Stream object around it, where this torch has the (private) call: 0.6 us, not 3
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None and torch.cuda.is_initialized():
+        return ctypes.c_void_p(raw(torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
