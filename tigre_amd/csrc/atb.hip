@@ -199,8 +199,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(atb_waves(k
 // root).
 //
 // The window is the projection of the patch's corners: u and v are
-// linear-fractional in the voxel position (the source is never inside the
-// patch), so over the patch their extremes lie at corners; kWinMargin (or
+// linear-fractional in the voxel position, so over a patch on one side of the
+// source their extremes lie at corners (a patch on both sides, where the
+// source is among the voxels, counts as one that does not fit); kWinMargin (or
 // four roundings of the coordinate, on detectors beyond 32768) covers the
 // rounding of the other lanes.  A view whose window does not fit is gathered
 // from global memory; both paths read the same quads with the same
@@ -333,7 +334,7 @@ __device__ __forceinline__ void atb_lds_block(const float* __restrict__ proj, in
     float wrow = 0.0f;
     auto windows = [&](int first) {
         const ViewParams w = view_params(views[min(first + lane, nviews - 1)]);
-        float vlo = __builtin_inff(), vhi = -vlo, ulo = hu, uhi = 0.0f;
+        float vlo = __builtin_inff(), vhi = -vlo, ulo = hu, uhi = 0.0f, dlo = vlo, dhi = vhi;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             float pu, pv0, dpv;
@@ -342,6 +343,8 @@ __device__ __forceinline__ void atb_lds_block(const float* __restrict__ proj, in
             const float pv1 = fmaf((float)(kG - 1), dpv, pv0);
             vlo = fminf(vlo, fminf(pv0, pv1));
             vhi = fmaxf(vhi, fmaxf(pv0, pv1));
+            dlo = fminf(dlo, dpv);
+            dhi = fmaxf(dhi, dpv);
             pu = __builtin_amdgcn_fmed3f(pu, 0.0f, hu);
             ulo = fminf(ulo, pu);
             uhi = fmaxf(uhi, pu);
@@ -353,7 +356,9 @@ __device__ __forceinline__ void atb_lds_block(const float* __restrict__ proj, in
         wsrc = (unsigned)r0 * rowb + (unsigned)c0 * 16u;
         wlds = -c0 * 16;
         wrow = (float)r0;
-        wblocks = r1 - r0 < kWinRows && c1 - c0 < kWinCols ? (r1 - r0 + 2) >> 1 : 0;
+        // (steps of one sign: the patch lies on one side of the source)
+        const bool fits = r1 - r0 < kWinRows && c1 - c0 < kWinCols && dlo * dhi > 0.0f && dhi - dlo < __builtin_inff();
+        wblocks = fits ? (r1 - r0 + 2) >> 1 : 0;
         if (wblocks > 0 && vlo >= mv && vhi <= hv - mv) wblocks += 32;
     };
     // Issues the copy of view p's window, the 2 x 32 blocks shared out over the wavefronts (the quads past the
