@@ -637,6 +637,12 @@ __device__ __forceinline__ bf16x8 tr_frag(const char* lo, const char* hi) {
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// A fragment with each pair of voxels masked.
+__device__ __forceinline__ bf16x8 masked(bf16x8 f, unsigned m0, unsigned m1, unsigned m2, unsigned m3) {
+    const uint4 u = __builtin_bit_cast(uint4, f);
+    return __builtin_bit_cast(bf16x8, make_uint4(u.x & m0, u.y & m1, u.z & m2, u.w & m3));
+}
+
 // A 16-byte chunk (channels 8 c .. 8 c + 7) of a voxel, or zeros for off < 0.
 template <int kIn>
 __device__ __forceinline__ uint4 load_chunk(const void* __restrict__ plane, int off, int c) {
@@ -692,6 +698,12 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2, 2
         const int zc = (u / (segW * tilesY)) % chunksZ;
         const long long n = u / (segW * tilesY * chunksZ);
         const int za = zc * zchunk, zb = min(za + zchunk, D);
+        // x voxels that no dy voxel of a tap meets are left out, not multiplied with the zeros around dy (an infinite one
+        // would make the tap NaN): here the one that dx = -1 pairs with voxel W, in a segment that W ends
+        unsigned edge_x[4];
+        const int past = W - xs - 8 * q;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) edge_x[j] = past == 2 * j ? 0xffff0000u : past == 2 * j + 1 ? 0x0000ffffu : ~0u;
         // this thread's chunks of a staged plane: voxel offsets from the tile's first row (-1: zero)
         int sx[kWgXIters], sd[kWgDIters];
 #pragma unroll
@@ -765,17 +777,22 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
                     for (int d = 0; d < 3; ++d)
                         a[d] = tr_frag(lx + r * (kWgXW * 64) + xo[d][0], lx + r * (kWgXW * 64) + xo[d][1]);
+                    a[0] = masked(a[0], edge_x[0], edge_x[1], edge_x[2], edge_x[3]);
+                    // (the volume's first row meets no dy row of the taps dy = 1, its last none of dy = -1)
+                    const int row = y0 + half * (kWgRows / 2) + r;
 #pragma unroll
                     for (int dz = 0; dz < 3; ++dz) {
                         b[dz][(r + 2) % 3] =
                             tr_frag(ld[dz] + (r + 2) * 2048 + po[0], ld[dz] + (r + 2) * 2048 + po[1]);
                         if (!on[dz]) continue;  // uniform
 #pragma unroll
-                        for (int dyy = 0; dyy < 3; ++dyy)  // tap dy = dyy - 1 reads dy row r - dy, halo'd index r + 2 - dyy
+                        for (int dyy = 0; dyy < 3; ++dyy) {  // tap dy = dyy - 1 reads dy row r - dy, halo'd index r + 2 - dyy
+                            if ((dyy == 0 && row == H - 1) || (dyy == 2 && r == 0 && row == 0)) continue;  // uniform
 #pragma unroll
                             for (int d = 0; d < 3; ++d)
                                 acc[dz * 9 + dyy * 3 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                                     a[d], b[dz][(r + 2 - dyy) % 3], acc[dz * 9 + dyy * 3 + d], 0, 0, 0);
+                        }
                     }
                     if (ih == 0)
                         acc[27] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[1][(r + 1) % 3], acc[27], 0, 0, 0);
