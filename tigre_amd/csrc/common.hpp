@@ -268,6 +268,15 @@ constexpr int kFilterMinLog = 6, kFilterMaxLog = 12;
 int launch_filter_rows(const float* in, const float* weight, const float* response, float* out, long long rows, int nV,
                        int nU, int log2_len, hipStream_t stream);
 int launch_cosine_weight(float* w, int nV, int nU, double dV, double dU, double dsd, hipStream_t stream);
+struct TvParams {
+    const float* prior;  // PICCS prior image
+    float inv_delta;     // AwTV 1 / delta
+    float ratio;         // PICCS prior ratio
+};
+// TV steps by LDS tiles (tv_tiles.hip): an iteration writes the partial sums of tv_tile_count() tiles and one scale.
+long long tv_tile_count(long nx, long ny, long nz);
+int launch_tv_tile_iteration(int kind, const float* src, float* out, const TvParams& tp, int nx, int ny, int nz,
+                             float alpha, double norm_eps, double* partial, float* scale, hipStream_t stream);
 int run_pocs_tv(const float* img, float* dst, float alpha, long nx, long ny, long nz, int maxiter,
                 hipStream_t stream);
 int run_aw_pocs_tv(const float* img, float* dst, float alpha, float delta, long nx, long ny, long nz, int maxiter,

@@ -10,12 +10,17 @@
 // exponential as the reference's __expf), so each n is
 // computed once per voxel instead of four times.  An iteration needs the norm
 // of the whole g before it can step, f' = f - alpha / sqrt(sum g^2 + norm_eps)
-// g, and is one pass all the same: the pass that makes f' from f also sums g^2
-// of f' for the next step (FP32 over eight voxels, FP64 beyond), and the next
-// pass adds up the workgroups' sums in a fixed order at its start, every
-// wavefront for itself.  A first pass only sums, the last only steps: no host
-// round trip for the norm, maxiter + 1 launches, 8 bytes of traffic per voxel
-// and iteration.
+// g.  Three forms, chosen by a rule on the sizes (run_tv_descent):
+//   one pass   makes f' from f and also sums g^2 of f' for the next step (FP32
+//              over eight voxels, FP64 beyond); the next pass adds up the
+//              workgroups' sums in a fixed order at its start, every wavefront for
+//              itself.  A first pass only sums, the last only steps: maxiter + 1
+//              launches, 8 bytes of traffic per voxel and iteration;
+//   two passes a pass for the norm and one for the step: 2 maxiter launches, 12
+//              bytes;
+//   LDS tiles  (tv_tiles.hip) two passes and a reduction: 3 maxiter launches, 12
+//              bytes.
+// None has a host round trip for the norm.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -32,12 +37,6 @@ template <int k>
 using Int = std::integral_constant<int, k>;
 constexpr int kTvBatch = 6;                                  // rows whose chains are interleaved
 constexpr int kTvBlocks = 1024;                              // workgroups of a pass, at most
-
-struct TvParams {
-    const float* prior;  // PICCS prior image
-    float inv_delta;     // AwTV 1 / delta
-    float ratio;         // PICCS prior ratio
-};
 
 // Workgroup sum of one double per lane (wavefront shuffles, then LDS), in every thread.
 __device__ inline double block_sum(double v) {
@@ -415,23 +414,37 @@ int run_tv_descent(const float* img, float* dst, float alpha, const TvParams& tp
     const bool small = ntx * ((ny + 7) / 8) * ((nz + 3) / 4) < 1024;
     const int rows = small ? 2 : 8;
     const long long nty = (ny + rows - 1) / rows, column = ntx * nty;
-    // A pass that takes the norm too evaluates n on 20 rows for 8 and 4 planes more a chunk, a pass for each on 18 and 2,
-    // and moves 8 bytes a voxel instead of 12.  Two passes pay while the Infinity Cache serves them (us for 20
-    // iterations, one and two passes: TV 150 x 140 x 160 415 and 374, 200^3 587 and 578, 320^3 1578 and 1650, 512^3 6297
-    // and 8112; PICCS 200^3 1030 and 950, 300^3 2510 and 2396, 400^3 5775 and 6643), and always for AwTV, which
-    // spends most on the weights' exponentials (240 x 230 x 250 1374 and 1092).
-    const bool fused = small || (kKind == 0 && n > (1u << 23)) || (kKind == 2 && n > (1u << 25));
+    // Three forms.  A pass that takes the norm too evaluates n on 20 rows for 8 and 4 planes more a chunk, a pass for each
+    // on 18 and 2, and moves 8 bytes a voxel instead of 12: one pass pays where the Infinity Cache no longer serves two
+    // and the chunks are not mostly halo (us an iteration, one and two passes: TV 250^3 47.3 and 45.0, 320^3 80.2 and 80.4,
+    // 512^3 315 and 406, 8 x 2048^2 108 and 95, 16 x 2048^2 206 and 225; PICCS 250^3 88 and 80, 300^3 125 and 120, 384^3
+    // 251 and 285), and never for AwTV, which spends most on the weights' exponentials (240 x 230 x 250 69 and 55).
+    // LDS tiles (tv_tiles.hip) take 1.2 to 1.5 times a wavefront tile's time for a column and plane, but have no halo to
+    // speak of: they serve AwTV where wavefront tiles fill the columns badly (LDS tiles and two passes: 250^3 59 and 68,
+    // 256^3 60 and 68, 384^3 192 and 198, 64 x 1024^2 226 and 248; 280^3 100 and 80, 320^3 123 and 111, 400^3 254 and 228),
+    // and the others on slabs of few planes (LDS tiles and the better of the rest: TV 16 x 1024^2 46 and 50, 16 x 2048^2
+    // 189 and 206, 8 x 2048^2 96 and 95; PICCS 8 x 1024^2 50 and 52, 16 x 2048^2 326 and 383, 4 x 1024^2 35 and 33).
+    const bool fused = small || (kKind == 0 && n > (1u << 24) && nz > 8) || (kKind == 2 && n > (1u << 25));
     const int chunk = small ? (int)std::max(2LL, ceil_div(nz, std::max(1LL, 3072 / column)))
                             : tv_chunk(column, nz, fused ? 4 : 2);
+    bool tiles = false;
+    if (!small) {
+        // evaluations of n an iteration, by LDS tiles and by two passes
+        const double by_tiles = 16.0 * (double)(ceil_div(nx, 128) * 128 * nty) * (double)(nz + ceil_div(nz, 16));
+        const double by_passes = 18.0 * (double)(64 * column) * (double)(nz + 2 * ceil_div(nz, tv_chunk(column, nz, 2)));
+        const bool cheap = tv_tile_count(nx, ny, nz) >= 960 && by_tiles < 0.8 * by_passes;
+        tiles = cheap && (kKind == 0 ? nz > 8 && nz <= 32 && n >= (1u << 24) : kKind == 1 ? nz >= 2 : nz >= 8 && nz <= 32);
+    }
     const long long ntiles = column * ((nz + chunk - 1) / chunk);
     TIGRE_REQUIRE(ntiles < (1LL << 30), "image too large");
     const int nblocks = (int)std::min((long long)kTvBlocks, (ntiles + kTvWaves - 1) / kTvWaves);
+    const size_t npartial = tiles ? (size_t)tv_tile_count(nx, ny, nz) + 1 : 2 * kTvBlocks;
     StreamScratch scratch(stream);
     float* buf[2] = {nullptr, nullptr};
     double* partial[2] = {nullptr, nullptr};
     TIGRE_CHECK(scratch.alloc(&buf[0], n * sizeof(float)));
     TIGRE_CHECK(scratch.alloc(&buf[1], n * sizeof(float)));
-    TIGRE_CHECK(scratch.alloc(&partial[0], 2 * kTvBlocks * sizeof(double)));
+    TIGRE_CHECK(scratch.alloc(&partial[0], npartial * sizeof(double)));
     partial[1] = partial[0] + kTvBlocks;
     const float* src = img;
     int cur = 0;
@@ -439,6 +452,13 @@ int run_tv_descent(const float* img, float* dst, float alpha, const TvParams& tp
         const bool last = it == maxiter - 1;
         float* o = (last && dst != img) ? dst : buf[cur];
         KernelTimerScope timer(TIGRE_KERNEL_POCS_TV, stream);
+        if (tiles) {
+            TIGRE_CHECK(launch_tv_tile_iteration(kKind, src, o, tp, (int)nx, (int)ny, (int)nz, alpha, norm_eps, partial[0],
+                                                 reinterpret_cast<float*>(partial[0] + npartial - 1), stream));
+            src = o;
+            cur ^= 1;
+            continue;
+        }
 #define TIGRE_TV(C, U, N)                                                                                          \
     hipLaunchKernelGGL((tv_kernel<kKind, C, U, N>), dim3((unsigned)nblocks), dim3(kTvThreads), 0, stream, src, o, tp, \
                        (int)nx, (int)ny, (int)nz, (int)ntx, (int)nty, chunk, (int)ntiles, alpha, norm_eps,          \
