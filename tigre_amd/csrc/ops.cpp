@@ -43,6 +43,16 @@ BeamClass beam_class(const HostGeometry& g, const FwdView& w) {
     return k;
 }
 
+// Whether the slab box of a 32 x 32 tile in one view, on the axis, fits eight planes of the beam kernel's LDS buffer: a
+// ray at 45 degrees moves by a plane's width and seven columns go to alignment, and by about a slice in z, with its taps.
+bool wide_tile_fits(const HostGeometry& g) {
+    double mag = 0.0;
+    for (int i = 0; i < g.nangles; ++i) mag = std::max(mag, g.parallel ? 1.0 : g.DSO[i] / g.DSD[i]);
+    const double columns = 32.0 * g.dDetec[0] * mag / std::min(g.dVoxel[0], g.dVoxel[1]) + 8.0 + 7.0;
+    const double rows = 32.0 * g.dDetec[1] * mag / g.dVoxel[2] + 1.2 + 3.0;
+    return columns * rows * 8.0 <= 9216.0;
+}
+
 }  // namespace
 
 void build_forward_records(const HostGeometry& g, bool interp, int views_per_group, ForwardRecords* rec) {
@@ -83,7 +93,7 @@ void build_forward_records(const HostGeometry& g, bool interp, int views_per_gro
     double tile_mm = INFINITY, reach_mm = 0.0;
     for (int i = 0; i < g.nangles; ++i) {
         const double mag = g.parallel ? 1.0 : g.DSO[i] / g.DSD[i];
-        tile_mm = std::min(tile_mm, 16.0 * g.dDetec[0] * mag);  // the beam kernel's 16-pixel tile at the axis
+        tile_mm = std::min(tile_mm, 16.0 * g.dDetec[0] * mag);  // 16 pixels, the width of a wavefront's unit, at the axis
         reach_mm = std::max(reach_mm, std::hypot(g.offOrig[3 * i], g.offOrig[3 * i + 1]));
     }
     reach_mm += 0.5 * std::hypot(g.sVoxel[0], g.sVoxel[1]);
@@ -120,14 +130,18 @@ void build_forward_records(const HostGeometry& g, bool interp, int views_per_gro
     // views 25.3 against 26.4 ms; a ragged 200^3 volume with 4-degree spacing, whose 16 x 16 boxes do not fit eight
     // planes, 0.68 against 0.74 ms).  Groups of fewer than four views leave view slots empty, and the tile grows to
     // 32 x 16 where that keeps a workgroup for every CU (a single view of a 256 x 256 detector in 64 workgroups
-    // measured 0.116 against 0.058 ms in 16 x 16 tiles).  It grows no further: with one view a group half of the
-    // wavefronts then only load, but the box is half that of a 64 x 16 or 32 x 32 tile and takes more planes
-    // (Siddon, 227 x 227 x 154, 20 views 0.32 against 0.48 and 0.40 ms, 320^3, 24 views 1.05 against 1.28 and 1.19;
-    // interpolated, 256^3, 20 views 1.04 against 1.21 in 32 x 32, 384^3, 24 views 3.71 against 4.09).
+    // measured 0.116 against 0.058 ms in 16 x 16 tiles).  With one view a group that leaves half of the wavefronts to
+    // load only, but the box is half that of a 32 x 32 tile and takes more planes: the tile grows to 32 x 32 where its
+    // box still fits eight planes, that is with pixels below three quarters of a voxel (times of 32 x 16 and 32 x 32, by
+    // pixel over voxel on the axis; Siddon, 320^3, 24 views 1: 1.18 and 1.26 ms, 0.8: 1.40 and 1.50, 0.65: 1.85 and
+    // 1.59, 0.4: 4.36 and 3.15; interpolated, 512^3, 40 views 1: 16.7 and 19.7, 0.8: 21.3 and 21.0, 0.65: 30.7 and 27.9,
+    // 0.4: 46.1 and 38.8).
     int most = 0;
     for (int k = 0; k < rec->ngroups(); ++k) most = std::max(most, rec->groups[4 * k + 1]);
     rec->shape = interp ? BeamShape{1, 4} : BeamShape{2, 2};
     if (most <= 2 && beam_job_blocks(g, rec->ngroups(), BeamShape{2, 4}) >= 256) rec->shape = BeamShape{2, 4};
+    if (most == 1 && beam_job_blocks(g, rec->ngroups(), BeamShape{2, 8}) >= 256 && wide_tile_fits(g))
+        rec->shape = BeamShape{2, 8};
 }
 
 namespace {
