@@ -336,7 +336,7 @@ def main():
     else:
         dom, dom_ms, dom_b = "ax_siddon", k_siddon, b_ax
     achieved = dom_b / (dom_ms * 1e-3) / 1e9
-    traffic = measured_traffic(dom)
+    traffic = measured_traffic(dom) if (n, nviews) == (512, 360) else None
 
     result = {
         "metric": "Ax+Atb Gupdates/s (Siddon + FDK, cone beam)",
@@ -355,7 +355,11 @@ def main():
             n, nviews, n, n), "nVoxel": [n, n, n], "nViews": nviews, "nDetector": [n, n],
             "DSO_mm": 1000.0, "DSD_mm": 1536.0},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+                     "achieved_is": "model bytes per launch / kernel time: an effective rate, not the HBM's",
+                     "traffic": traffic,
+                     "traffic_gb_s": round(traffic / (dom_ms * 1e-3) / 1e9, 1) if traffic else None,
+                     "traffic_frac": round(traffic / (dom_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
                      "model_bytes_per_launch": dom_b, "kernel_ms": round(dom_ms, 3)},
         "ops_ms": {"ax_siddon": round(ax_ms, 3), "atb_fdk": round(atb_ms, 3), "ax_interpolated": round(interp_ms, 3),
                    "atb_matched": round(matched_ms, 3)},

@@ -188,14 +188,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(atb_waves(k
 // of view p, into the window of view p - 1, so it overlaps the updates; one
 // barrier a view both publishes a window and frees the other.
 //
-// What bounds it: vector issue (8.8 instructions an update: step, conversion,
-// fraction, address, three for the sample, one for the sum, and 0.8 for the
-// column) next to LDS reads (one ds_read_b128 an update, 5.4 clocks with
+// What bounds it: vector issue (9.3 instructions an update, 8.8 of them in the
+// slice loop: row, conversion, fraction, address, three for the sample, one for
+// the sum, and 0.8 for the column) next to LDS reads (one ds_read_b128 an update, 5.4 clocks with
 // conflicts).  A window per wavefront (8 x 8 columns) copied 2.2 times the
 // quads, and L2 could not feed them: 15.3 to 17.5 ms at 512^3, 360 views,
-// depending on how many wavefronts shared a cache.  512^3: 17.2 -> 10.5 ms;
+// depending on how many wavefronts shared a cache.  512^3: 17.2 -> 10.9 ms;
 // 256^3, 180 views: 1.28 -> 0.79 ms; matched weight, 237 x 256 x 191, 180
-// views: 1.15 -> 1.05 ms (18 instructions an update, one of them a reciprocal
+// views: 1.15 -> 1.05 ms (18.7 instructions an update, one of them a reciprocal
 // root).
 //
 // The window is the projection of the patch's corners: u and v are

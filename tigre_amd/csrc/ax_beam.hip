@@ -1,8 +1,10 @@
 // Beam-staged forward projectors for gfx950.
 //
-// A 1024-thread workgroup traces the rays of a detector tile (1024 rays: 32 x 8 pixels in four views, 64 x 16
-// in one, ...) in up to four views that share a principal axis P (the horizontal axis, x or y, along
-// which their rays advance fastest) and its direction.  Their rays form a thin
+// A 1024-thread workgroup traces the rays of a detector tile in up to four views that share a principal axis P (the
+// horizontal axis, x or y, along which their rays advance fastest) and its direction.  A wavefront takes 16 x 4
+// pixels of one view; the tile (BeamShape) is 32 x 8 pixels (Siddon) or 16 x 16 (interpolated) in four views, 32 x 16
+// in two or one, 32 x 32 in one (build_forward_records chooses).  Wavefronts without a view, half of them where a
+// 32 x 16 tile has one view, only copy.  Their rays form a thin
 // beam.  The workgroup sweeps the volume along P in slabs of a few planes; for
 // each slab it copies the box of voxels the beam crosses into LDS (16-byte
 // loads of rows of a re-laid-out copy of the volume), and every ray walks its
@@ -231,9 +233,9 @@ __device__ inline bool walk(RayWalk& r, const float* __restrict__ base, unsigned
 // degree diagonal, about 4 % of them at a fan angle of 15 degrees) and for the flat ones (a pixel row or column about
 // the central one, where pixels are smaller than about 2^-12 of the source's distance).
 //
-// Measured at 512^3 voxels, 512^2 pixels, 360 views: 25.3 ms, 36.5 ms with the crossing walk alone; 23 VALU
+// Measured at 512^3 voxels, 512^2 pixels, 360 views: 25.8 ms, 36.5 ms with the crossing walk alone; 23.5 VALU
 // instructions per ray and plane (33.8 before), 3.4 cycles each (most pairs of an FMA and another operation
-// issue together), and 5 TB/s of copies.  What is scalar or serial in the slab loop counts as much:
+// issue together), and 5.7 TB/s of copies.  The second walk for infinite voxels and the flat rays' walk are 2 % of it.  What is scalar or serial in the slab loop counts as much:
 // with the slabs' addresses formed in the loop instead of read from a table the same walk took 30.5 ms.  Two rays per lane
 // with half the wavefronts moved 40 % less and were slower (33 ms).
 struct PlaneRay {

@@ -230,7 +230,9 @@ __global__ __launch_bounds__(kTvThreads, kKind == 2 ? 2 : 3) void tv_kernel(cons
                 }
                 // n_z + n_y.  n is discontinuous where all differences vanish, so another rounding of g than the one results
                 // have always had moves single voxels by 1e-3 of the range after some iterations: here that is the
-                // rounded product, and in every sixteenth plane the fused one.
+                // rounded product, and in every sixteenth plane the fused one.  (No more exact than one form in all planes,
+                // and the bits depend on where the image starts in z: the rounded product throughout moved one of 25
+                // images of 256^3 by 1.6e-3, the same n_z for the voxel and its neighbour 19 of 80 images by up to 9.4e-3.)
                 float zy[kB];
                 if (NF == 1 && (z & 15) == 0) {
 #pragma unroll
@@ -655,7 +657,9 @@ __global__ __launch_bounds__(64 * kRofWaves) void rof_kernel(const float* __rest
                     q.z = fmaf(t2 * idz, !kEdge || z < D ? un[r] - u : 0.0f, p.z);
                     q.y = fmaf(t2 * idy, !kEdge || y + 1 < ny ? uy - u : 0.0f, p.y);
                     q.x = fmaf(t2 * idx, x_last ? 0.0f : dx, p.x);
-                    // 1 / max(1, |q|); q = 0 gives 1
+                    // 1 / max(1, |q|); q = 0 gives 1.  Errors from FP64 as with a square root and divisions, geometric means
+                    // over 24 cases a spacing: 1.0924e-7 and 1.0943e-7 (spacing 1), 1.5549e-7 and 1.5562e-7 (0.3 to 0.9);
+                    // 150 x 181 x 170, 50 iterations: 669 and 1249 us.
                     const float inv = fminf(1.0f, __builtin_amdgcn_rsqf(fmaf(q.z, q.z, fmaf(q.y, q.y, q.x * q.x))));
                     q.z *= inv;
                     q.y *= inv;
