@@ -4,8 +4,8 @@
 // horizontal axis, x or y, along which their rays advance fastest) and its direction.  A wavefront takes 16 x 4
 // pixels of one view; the tile (BeamShape) is 32 x 8 pixels (Siddon) or 16 x 16 (interpolated) in four views, 32 x 16
 // in two or one, 32 x 32 in one (build_forward_records chooses).  Wavefronts without a view, half of them where a
-// 32 x 16 tile has one view, only copy.  Their rays form a thin
-// beam.  The workgroup sweeps the volume along P in slabs of a few planes; for
+// 32 x 16 tile has one view, only copy.
+// The rays form a thin beam.  The workgroup sweeps the volume along P in slabs of a few planes; for
 // each slab it copies the box of voxels the beam crosses into LDS (16-byte
 // loads of rows of a re-laid-out copy of the volume), and every ray walks its
 // voxels inside the slab from LDS.  The gathers of
@@ -235,9 +235,10 @@ __device__ inline bool walk(RayWalk& r, const float* __restrict__ base, unsigned
 //
 // Measured at 512^3 voxels, 512^2 pixels, 360 views: 25.8 ms, 36.5 ms with the crossing walk alone; 23.5 VALU
 // instructions per ray and plane (33.8 before), 3.4 cycles each (most pairs of an FMA and another operation
-// issue together), and 5.7 TB/s of copies.  The second walk for infinite voxels and the flat rays' walk are 2 % of it.  What is scalar or serial in the slab loop counts as much:
-// with the slabs' addresses formed in the loop instead of read from a table the same walk took 30.5 ms.  Two rays per lane
-// with half the wavefronts moved 40 % less and were slower (33 ms).
+// issue together), and 5.7 TB/s of copies.  The second walk for infinite voxels and the flat rays' walk are 2 %
+// of it.  What is scalar or serial in the slab loop counts as much: with the slabs' addresses formed in the loop
+// instead of read from a table the same walk took 30.5 ms.  Two rays per lane with half the wavefronts moved 40 %
+// less and were slower (33 ms).
 struct PlaneRay {
     unsigned long long A0, z0;  // mirrored A and z at the start of cell -1, 2^-32 voxel
     unsigned kA, kz;            // slopes, 2^-32 voxel
