@@ -253,13 +253,13 @@ struct PlaneRay {
 __device__ __forceinline__ float flat_slope(int nP) { return fmaxf(0x1p-9f / sqrtf((float)nP), 0x1p-6f / (float)nP); }
 
 // Mirrored position and slope on one axis of the line s0 + r a, from the start of cell -1, which the
-// sweep enters at parameter a0 and leaves da later; a ray parallel to the axis stays inside its voxel
-// (or on the border).
+// sweep enters at parameter a0 and leaves da later; a ray parallel to the axis stays inside its voxel,
+// or on the border that it is next to (the other one need not lie in the box).
 __device__ __forceinline__ void plane_axis(double s0, double r, double a0, double da, int n, unsigned long long& x0,
                                            unsigned& k, float& ik, int& step) {
     double x = s0 + r * a0, slope = r * da;
     step = 1;
-    if (r == 0.0) x = (s0 > 0.0 && s0 < (double)n) ? floor(s0) + 0.5 : -1.0;
+    if (r == 0.0) x = s0 <= 0.0 ? -1.0 : s0 >= (double)n ? (double)n : floor(s0) + 0.5;
     if (slope < 0.0) {
         x = (double)n - x;
         slope = -slope;
